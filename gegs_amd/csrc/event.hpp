@@ -26,7 +26,8 @@
 //     particle and no source record is left, or until every record is
 //     injected and few particles remain, which one tail launch then
 //     finishes, each particle with its descendants in one thread; the host
-//     reads the loop's state once per replay.
+//     reads the loop's state once per replay.  A run of few histories goes
+//     to the tail launch right after its injection.
 // Particles keep their Philox streams across banks, so every history follows
 // exactly the trajectory the plain kernel and the oracle give it.
 #pragma once
@@ -96,6 +97,7 @@ struct EventConfig {
     uint32_t inject = 6u << 20;      // primaries injected per refill
     uint32_t threshold = 6u << 20;   // refill when fewer particles are in flight
     uint32_t sweeps_per_graph = 4;
+    bool direct = true;              // a run of at most TAIL_DIRECT histories takes the tail launch at once
 };
 
 // Source records of one batch, as slices of every job (field) of the run:
@@ -779,9 +781,14 @@ __global__ void sweep_end(EvState *st, uint32_t threshold, uint32_t max_inject) 
 // as the plain kernel does, secondaries on a per-thread stack, interactions
 // in line.  A particle's trajectory does not depend on which kernel moves
 // it (each carries its stream), so the histories are the sweeps' own; a
-// suspended electron resumes from its banked step state.
+// suspended electron resumes from its banked step state.  It is bound by the
+// longest chain of dependent steps of one wavefront, so the particles are
+// spread over all resident wavefronts, a few lanes of each (plain_lanes):
+// 1 000 histories' last particles on the CT 1.71 -> 1.1 ms, 100 003 through
+// jaws and MLC 17.9 -> 12 ms against 64 lanes each.
 template <bool TAB, bool ADJ, bool GEN>
-__global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) tail_kernel(EvArgs a, float *stack, int depth) {
+__global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) tail_kernel(EvArgs a, float *stack, int depth,
+                                                                        uint32_t waves) {
     extern __shared__ float lds_env[];
     const uint32_t flip = a.st->flip;
     const int sp_in = bank_slot(P_PHOTON_STEP, flip, true);
@@ -790,7 +797,9 @@ __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) tail_kernel(EvArgs a
     vp.load(a, sp_in);
     ve.load(a, se_in);
     const uint32_t np = vp.total(), n = np + ve.total();
-    if (n == 0) return;
+    // each wavefront takes its share of the particles in its first lanes
+    const uint32_t lanes = plain_lanes(n, waves);
+    if (((blockIdx.x * blockDim.x) >> 6) * lanes >= n) return;   // nothing for any wavefront of the block
     Env env = a.env;
     env.fixes = kernel_fixes<GEN>(env.fixes);
     stage_env<TAB>(env, lds_env);
@@ -805,7 +814,8 @@ __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) tail_kernel(EvArgs a
     uint32_t pops[N_EVENTS];
 #pragma unroll
     for (int k = 0; k < N_EVENTS; ++k) pops[k] = 0;
-    for (uint32_t k = sink.tid; k < n; k += sink.stride) {
+    const uint32_t first = lane_id() < lanes ? (sink.tid >> 6) * lanes + lane_id() : n;
+    for (uint32_t k = first; k < n; k += (sink.stride >> 6) * lanes) {
         const bool photon = k < np;
         const uint32_t at = photon ? vp.slot_of(a, k) : ve.slot_of(a, k - np);
         uint32_t hist;
@@ -1081,6 +1091,14 @@ inline void launch_sweep(const EvArgs &a, const EventConfig &cfg, hipStream_t st
 }
 
 constexpr uint32_t TAIL_BLOCK = 128;
+// Histories of a run that the tail launch takes from the injection on, without
+// sweeps: up to 8192, 4 lanes of each resident wavefront.  A sweep of so few
+// particles takes as long as its slowest flight and there are at least 8
+// (two graph replays).  Kernel time with and without the sweeps: 1 000
+// histories on the CT 2.6 -> 1.5 ms, 4 096 2.8 -> 2.2 ms, 10 001 on water
+// 2.35 -> 1.65 ms and through jaws and MLC 12.8 -> 9.1 ms; at 16 384 on the CT
+// 3.2 against 3.4 ms, at 70 001 3.3 against 4.8 ms.
+constexpr uint32_t TAIL_DIRECT = 8192;
 constexpr int TAIL_DEPTH = 40;       // particles per thread's stack (the plain kernel's default)
 
 // threads of the tail launch: one per particle up to `tail`, whole blocks
@@ -1090,17 +1108,25 @@ inline uint32_t tail_threads(const EventConfig &cfg) {
 
 // The tail launch and the bookkeeping after it; `stack` holds
 // tail_threads(cfg) x TAIL_DEPTH particles.
+template <bool TAB, bool ADJ, bool GEN>
+inline void launch_tail_t(const EvArgs &a, const EventConfig &cfg, float *stack, hipStream_t stream) {
+    const uint32_t grid = tail_threads(cfg) / TAIL_BLOCK;
+    const size_t lds = flight_lds(a.env);
+    const uint32_t resident = resident_grid(tail_kernel<TAB, ADJ, GEN>, TAIL_BLOCK, lds);
+    const uint32_t waves = (grid < resident ? grid : resident) * (TAIL_BLOCK / 64);
+    hipLaunchKernelGGL((tail_kernel<TAB, ADJ, GEN>), dim3(grid), dim3(TAIL_BLOCK), lds, stream, a, stack, TAIL_DEPTH,
+                       waves);
+}
+
 template <bool GEN>
 inline void launch_tail_g(const EvArgs &a, const EventConfig &cfg, float *stack, hipStream_t stream) {
-    const dim3 g(tail_threads(cfg) / TAIL_BLOCK), b(TAIL_BLOCK);
-    const size_t lds = flight_lds(a.env);
     const bool adj = a.adj != nullptr;
     if (tab_in_lds(a.env)) {
-        if (adj) hipLaunchKernelGGL((tail_kernel<true, true, GEN>), g, b, lds, stream, a, stack, TAIL_DEPTH);
-        else hipLaunchKernelGGL((tail_kernel<true, false, GEN>), g, b, lds, stream, a, stack, TAIL_DEPTH);
+        if (adj) launch_tail_t<true, true, GEN>(a, cfg, stack, stream);
+        else launch_tail_t<true, false, GEN>(a, cfg, stack, stream);
     } else {
-        if (adj) hipLaunchKernelGGL((tail_kernel<false, true, GEN>), g, b, lds, stream, a, stack, TAIL_DEPTH);
-        else hipLaunchKernelGGL((tail_kernel<false, false, GEN>), g, b, lds, stream, a, stack, TAIL_DEPTH);
+        if (adj) launch_tail_t<false, true, GEN>(a, cfg, stack, stream);
+        else launch_tail_t<false, false, GEN>(a, cfg, stack, stream);
     }
     hipLaunchKernelGGL(tail_end, dim3(1), dim3(1), 0, stream, a.st);
 }
@@ -1206,9 +1232,14 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
     // group is captured once per argument set and replayed.
     const bool timed = bk.timing && cfg.sweeps_per_graph <= (uint32_t)EventBanks::MAX_TIMED;
     const SweepFork fork = cfg.sweep_streams == 2 ? bk.fork : SweepFork();
+    const bool use_tail = cfg.tail && !timed;
+    // a run this short goes to the tail launch at once: no sweeps, no graph
+    const uint32_t total = bk.h_plan->total;
+    const bool direct = use_tail && cfg.direct && total <= TAIL_DIRECT && total <= cfg.inject && total <= cfg.tail;
     if (timed) {
         e = bk.make_timing_events();
         if (e != hipSuccess) return e;
+    } else if (direct) {
     } else if (!bk.graph[0] || !same_args(a, bk.graph_args) || !same_cfg(cfg, bk.graph_cfg)) {
         bk.drop_graph();
         hipGraph_t g;
@@ -1223,9 +1254,30 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
         bk.graph_args = a;
         bk.graph_cfg = cfg;
     }
+    // The tail launch finishes the run once every record is injected and at
+    // most cfg.tail particles are in flight (not in a timed pass, whose
+    // photon steps must all be photon-kernel steps).
+    if (use_tail) {
+        const size_t need = (size_t)tail_threads(cfg) * TAIL_DEPTH * PART_WORDS;
+        if (bk.tail_floats < need) {
+            if (bk.tail_stack) (void)hipFree(bk.tail_stack);
+            bk.tail_stack = nullptr;
+            bk.tail_floats = 0;
+            e = hipMalloc(&bk.tail_stack, need * sizeof(float));
+            if (e != hipSuccess) return e;
+            bk.tail_floats = need;
+        }
+    }
     e = hipMemcpyAsync(bk.d_plan, bk.h_plan, sizeof(BatchPlan), hipMemcpyHostToDevice, stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(batch_begin, dim3(1), dim3(1), 0, stream, bk.st, 0u, bk.h_plan->total, cfg.threshold, cfg.inject);
+    if (direct) {
+        hipLaunchKernelGGL(inject_fill, dim3(cfg.grid), dim3(cfg.block), 0, stream, a);
+        launch_tail(a, cfg, bk.tail_stack, stream);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        // the plan's staging copy may be refilled once this returns
+        return hipStreamSynchronize(stream);
+    }
     // Two replays in flight: while the host waits for the flag of replay k,
     // replay k+1 is already queued, so the GPU does not idle during the host
     // round trip.  The replay queued after the last busy one finds every bank
@@ -1246,21 +1298,6 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
         if (r != hipSuccess) return r;
         return hipEventRecord(bk.done[slot], stream);
     };
-    // The tail launch finishes the run once every record is injected and at
-    // most cfg.tail particles are in flight (not in a timed pass, whose
-    // photon steps must all be photon-kernel steps).
-    const bool use_tail = cfg.tail && !timed;
-    if (use_tail) {
-        const size_t need = (size_t)tail_threads(cfg) * TAIL_DEPTH * PART_WORDS;
-        if (bk.tail_floats < need) {
-            if (bk.tail_stack) (void)hipFree(bk.tail_stack);
-            bk.tail_stack = nullptr;
-            bk.tail_floats = 0;
-            e = hipMalloc(&bk.tail_stack, need * sizeof(float));
-            if (e != hipSuccess) return e;
-            bk.tail_floats = need;
-        }
-    }
     auto tail_ready = [&](int slot) {
         const uint32_t *f = bk.h_flags + FLAG_WORDS * slot;
         // every record injected (src_next >= src_last, no injection planned), inflight

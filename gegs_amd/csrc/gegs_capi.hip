@@ -629,6 +629,15 @@ static int check_ready(gegs_ctx *c, const gegs_run_options *o) {
     return GEGS_OK;
 }
 
+// Batch rows held at once by a continuous run (bytes of per-batch dose rows).
+static constexpr size_t CONTINUOUS_TALLY_BYTES = (size_t)16 << 30;
+
+// dose rows of nvox doubles that fit `bytes`: at least one, at most one per batch
+static uint32_t batch_rows(size_t bytes, size_t nvox, uint32_t n_batches) {
+    const size_t fit = bytes / (nvox * sizeof(double));
+    return fit < 1 ? 1u : (fit < n_batches ? (uint32_t)fit : n_batches);
+}
+
 // the plain kernel instantiation for the record-table placement and the
 // options of the run (the general kernel for any of ENV_GENERAL)
 static void launch_plain(const PlainArgs &a, bool tab, uint32_t grid, uint32_t block, size_t lds, hipStream_t st) {
@@ -639,65 +648,104 @@ static void launch_plain(const PlainArgs &a, bool tab, uint32_t grid, uint32_t b
     else hipLaunchKernelGGL((plain_kernel<false, false>), dim3(grid), dim3(block), lds, st, a);
 }
 
+// blocks of the plain kernel that are resident at once
+static uint32_t plain_resident(const PlainArgs &a, bool tab, size_t lds) {
+    const bool gen = (a.env.fixes & ENV_GENERAL) != 0;
+    if (tab && gen) return resident_grid(plain_kernel<true, true>, PLAIN_BLOCK, lds);
+    if (tab) return resident_grid(plain_kernel<true, false>, PLAIN_BLOCK, lds);
+    if (gen) return resident_grid(plain_kernel<false, true>, PLAIN_BLOCK, lds);
+    return resident_grid(plain_kernel<false, false>, PLAIN_BLOCK, lds);
+}
+
+// The histories of a run, `rows` statistical batches per launch: each batch
+// has its own dose row, so one launch carries as many batches as there are
+// rows and the GPU drains once per launch, where a launch per batch ended
+// on its slowest history every time: 1e6 histories on the 128x128x100 CT in
+// ten batches 67 -> 33 ms, 1e4 57 -> 2.8 ms; without allocation on 60^3
+// water, 20 011 in ten batches 34 -> 2.4 ms.
+static void launch_plain_batches(PlainArgs a, const gegs_run_options *o, uint64_t nr, uint32_t rows, uint32_t *next,
+                                 uint32_t grid, uint32_t resident, bool tab, size_t lds, double *dose, double *dose2,
+                                 hipStream_t st) {
+    const uint32_t nb = o->n_batches;
+    const uint64_t waves = (uint64_t)(grid < resident ? grid : resident) * (PLAIN_BLOCK / 64);
+    a.run_first = o->first;
+    a.n_run = nr;
+    a.n_batches = nb;
+    uint32_t pass = 0;
+    for (uint32_t b = 0; b < nb; b += rows, ++pass) {
+        const uint32_t b1 = nb - b < rows ? nb : b + rows;
+        a.first = (uint32_t)(o->first + (nr * b) / nb);
+        a.last = (uint32_t)(o->first + (nr * b1) / nb);
+        a.batch0 = b;
+        a.next = next + pass;
+        a.lanes = plain_lanes(a.last - a.first, waves);
+        launch_plain(a, tab, grid, PLAIN_BLOCK, lds, st);
+        hipLaunchKernelGGL(fold_batches, dim3(2048), dim3(256), 0, st, a.dose, dose, dose2, a.nvox, (size_t)1, b1 - b);
+    }
+}
+
 int gegs_run_plain(gegs_ctx *c, const gegs_run_options *o, double *dose, double *dose2) {
     int rc = check_ready(c, o);
     if (rc) return rc;
     hipSetDevice(c->device);
-    rc = prepare_tallies(c, 1, c->nsrc);
+    const uint32_t rows = batch_rows(CONTINUOUS_TALLY_BYTES, c->nvox, o->n_batches);
+    rc = prepare_tallies(c, 1, c->nsrc, rows);
     if (rc) return rc;
     rc = upload_jobs(c, {c->field}, {0u});
     if (rc) return rc;
-    const uint32_t block = o->block_size ? o->block_size : 128;
-    if (block != 128) return fail(c, GEGS_ERR_ARG, "run_plain: block_size must be 128");
-    const uint32_t grid = o->grid_size ? o->grid_size : 2048;
+    const uint32_t block = o->block_size ? o->block_size : PLAIN_BLOCK;
+    if (block != PLAIN_BLOCK) return fail(c, GEGS_ERR_ARG, "run_plain: block_size must be 128");
+    PlainArgs a;
+    a.env = make_env(c, o->seed, 1);
+    const bool tab = c->nclass <= LDS_MAX_CLASSES;
+    const size_t lds = env_lds_bytes(c->nx, c->ny, c->nz, c->nclass, c->nmed, 1, tab);
+    const uint32_t resident = plain_resident(a, tab, lds);
+    // the threads take histories until none is left: blocks past the resident
+    // ones would start when the work is done
+    const uint32_t grid = o->grid_size ? o->grid_size : (resident < 2048 ? resident : 2048);
     const int depth = o->stack_depth ? (int)o->stack_depth : 40;
     const size_t nthreads = (size_t)grid * block;
     size_t have = c->stack_bytes / sizeof(float);
     HIPCHECK(c, realloc_dev(c->d_stack, have, nthreads * (size_t)depth * PART_WORDS), "hipMalloc stack");
     c->stack_bytes = have * sizeof(float);
-    PlainArgs a;
-    a.env = make_env(c, o->seed, 1);
     a.src = c->d_src;
     a.hist_offset = o->history_offset;
     a.stack = c->d_stack;
     a.depth = depth;
     a.dose = c->d_chunk;
+    a.nvox = c->nvox;
     a.hist_edep = c->hist_tally ? c->d_hist_edep : nullptr;
     a.hist_steps = c->hist_tally ? c->d_hist_steps : nullptr;
     a.counters = c->d_counters;
-    const bool tab = c->nclass <= LDS_MAX_CLASSES;
-    const size_t lds = env_lds_bytes(c->nx, c->ny, c->nz, c->nclass, c->nmed, 1, tab);
     hipEvent_t t0, t1;
     hipEventCreate(&t0);
     hipEventCreate(&t1);
     hipEventRecord(t0, c->stream);
-    const uint32_t nb = o->n_batches;
-    const uint64_t r0 = o->first, nr = o->count ? o->count : c->nsrc - o->first;
-    for (uint32_t b = 0; b < nb; ++b) {
-        a.first = (uint32_t)(r0 + (nr * b) / nb);
-        a.last = (uint32_t)(r0 + (nr * (b + 1)) / nb);
-        a.next = c->d_next + b;
-        launch_plain(a, tab, grid, block, lds, c->stream);
-        hipLaunchKernelGGL(fold_batch, dim3(2048), dim3(256), 0, c->stream, c->d_chunk, c->d_dose, c->d_dose2, c->nvox);
-    }
+    const uint64_t nr = o->count ? o->count : c->nsrc - o->first;
+    launch_plain_batches(a, o, nr, rows, c->d_next, grid, resident, tab, lds, c->d_dose, c->d_dose2, c->stream);
     hipEventRecord(t1, c->stream);
     HIPCHECK(c, hipGetLastError(), "launch plain_kernel");
     return finish_run(c, dose, dose2, t0, t1);
 }
 
+// Part of the no-alloc scratch that may hold dose rows of several batches; the
+// rest is for particle stacks (a 128x128x100 CT's five rows leave 616 blocks
+// of 40-deep stacks, one row 778).
+static constexpr size_t NOALLOC_ROW_BYTES = GEGS_NOALLOC_SCRATCH_BYTES / 4;
+
 // Layout of the no-alloc scratch for a run on nvox voxels: counters, batch
 // work counters, the field, its plan index, jaw polygons, leaf ends, the
-// batch dose row, then the particle stacks.
+// batch dose rows, then the particle stacks.
 struct NoallocLayout {
     size_t counters = 0, next = 256, field, plan, polys, ends, chunk, stack;
-    explicit NoallocLayout(size_t nvox) {
+    NoallocLayout(size_t nvox, uint32_t rows) {
         auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
         field = up(next + 4096 * sizeof(uint32_t));
         plan = up(field + sizeof(gegs_field));
         polys = up(plan + sizeof(uint32_t));
         ends = up(polys + 32 * sizeof(gegs_float2));
         chunk = up(ends + (size_t)GEGS_MLC_LEAVES * 34 * sizeof(gegs_float2));
-        stack = up(chunk + nvox * sizeof(double));
+        stack = up(chunk + nvox * rows * sizeof(double));
     }
 };
 
@@ -711,17 +759,24 @@ int gegs_run_plain_noalloc(gegs_ctx *c, const gegs_run_options *o, double *dose,
     HIPCHECK(c, hipSetDevice(c->device), "set device");
     unsigned char *base = scratch_of(c->device);
     if (!base) return fail(c, GEGS_ERR_DEVICE, "run_plain_noalloc: no scratch address for this device");
-    const uint32_t block = o->block_size ? o->block_size : 128;
-    if (block != 128) return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: block_size must be 128");
+    const uint32_t block = o->block_size ? o->block_size : PLAIN_BLOCK;
+    if (block != PLAIN_BLOCK) return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: block_size must be 128");
     const int depth = o->stack_depth ? (int)o->stack_depth : 40;
-    const NoallocLayout L(c->nvox);
+    // an explicit grid keeps the room for stacks that one row leaves
+    const uint32_t rows = o->grid_size ? 1u : batch_rows(NOALLOC_ROW_BYTES, c->nvox, o->n_batches);
+    const NoallocLayout L(c->nvox, rows);
     const size_t per_block = (size_t)block * depth * PART_WORDS * sizeof(float);
     const size_t cap = GEGS_NOALLOC_SCRATCH_BYTES;
     if (L.stack + per_block > cap)
         return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: the phantom's dose row and one block of particle stacks "
                                      "exceed the scratch size (GEGS_NOALLOC_SCRATCH_BYTES)");
     const size_t fit = (cap - L.stack) / per_block;
-    uint32_t grid = 2048;
+    PlainArgs a;
+    a.env = make_env(c, o->seed, 1);
+    const bool tab = c->nclass <= LDS_MAX_CLASSES;
+    const size_t lds = env_lds_bytes(c->nx, c->ny, c->nz, c->nclass, c->nmed, 1, tab);
+    const uint32_t resident = plain_resident(a, tab, lds);
+    uint32_t grid = resident < 2048 ? resident : 2048;
     if (o->grid_size) {
         if (o->grid_size > fit)
             return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: grid_size x stack_depth exceeds the scratch size");
@@ -751,11 +806,9 @@ int gegs_run_plain_noalloc(gegs_ctx *c, const gegs_run_options *o, double *dose,
     // the scratch keeps the previous call's contents: clear what starts at zero
     hipLaunchKernelGGL(fill_zero_u64, dim3(1), dim3(64), 0, c->stream, counters, (size_t)16);
     hipLaunchKernelGGL(fill_zero_u32, dim3(16), dim3(256), 0, c->stream, next, (size_t)4096);
-    hipLaunchKernelGGL(fill_zero, dim3(2048), dim3(256), 0, c->stream, chunk, c->nvox);
+    hipLaunchKernelGGL(fill_zero, dim3(2048), dim3(256), 0, c->stream, chunk, c->nvox * rows);
     hipLaunchKernelGGL(fill_zero, dim3(2048), dim3(256), 0, c->stream, dose, c->nvox);
     hipLaunchKernelGGL(fill_zero, dim3(2048), dim3(256), 0, c->stream, dose2, c->nvox);
-    PlainArgs a;
-    a.env = make_env(c, o->seed, 1);
     a.env.fields = reinterpret_cast<const gegs_field *>(base + L.field);
     a.env.jaws = reinterpret_cast<const gegs_float2 *>(base + L.polys);
     a.env.endnodes = reinterpret_cast<const gegs_float2 *>(base + L.ends);
@@ -764,20 +817,12 @@ int gegs_run_plain_noalloc(gegs_ctx *c, const gegs_run_options *o, double *dose,
     a.stack = reinterpret_cast<float *>(base + L.stack);
     a.depth = depth;
     a.dose = chunk;
+    a.nvox = c->nvox;
     a.hist_edep = nullptr;
     a.hist_steps = nullptr;
     a.counters = counters;
-    const bool tab = c->nclass <= LDS_MAX_CLASSES;
-    const size_t lds = env_lds_bytes(c->nx, c->ny, c->nz, c->nclass, c->nmed, 1, tab);
-    const uint32_t nb = o->n_batches;
-    const uint64_t r0 = o->first, nr = o->count ? o->count : c->nsrc - o->first;
-    for (uint32_t b = 0; b < nb; ++b) {
-        a.first = (uint32_t)(r0 + (nr * b) / nb);
-        a.last = (uint32_t)(r0 + (nr * (b + 1)) / nb);
-        a.next = next + b;
-        launch_plain(a, tab, grid, block, lds, c->stream);
-        hipLaunchKernelGGL(fold_batch, dim3(2048), dim3(256), 0, c->stream, chunk, dose, dose2, c->nvox);
-    }
+    const uint64_t nr = o->count ? o->count : c->nsrc - o->first;
+    launch_plain_batches(a, o, nr, rows, next, grid, resident, tab, lds, dose, dose2, c->stream);
     HIPCHECK(c, hipGetLastError(), "launch plain_kernel");
     HIPCHECK(c, hipStreamSynchronize(c->stream), "run");
     unsigned long long h[16];
@@ -805,9 +850,6 @@ struct JobSpec {
 // Event-queued transport of every job in one loop: each batch holds the
 // b-th of n_batches equal slices of every job, so that every batch is an
 // independent sample of every plan's dose.
-// Batch rows held at once by a continuous run (bytes of per-batch dose rows).
-static constexpr size_t CONTINUOUS_TALLY_BYTES = (size_t)16 << 30;
-
 static int run_event_jobs(gegs_ctx *c, const gegs_run_options *o, const std::vector<gegs_field> &fields,
                           const std::vector<JobSpec> &jobs, uint32_t n_plans, uint64_t n_slots, double *dose,
                           double *dose2, const BeamletArgs &bl = BeamletArgs(), bool dev_out = false) {
@@ -1016,6 +1058,7 @@ int gegs_set_tuning(gegs_ctx *c, const gegs_tuning *t) {
     if (!c) return GEGS_ERR_ARG;
     EventConfig cfg;
     if (t) {
+        cfg.direct = false;   // a caller's shape of the sweeps holds for runs of any length
         if (t->block) cfg.block = t->block;
         if (t->flight_block) cfg.flight_block = t->flight_block;
         if (t->refill_min) cfg.refill_min = t->refill_min;

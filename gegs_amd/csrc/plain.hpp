@@ -11,6 +11,7 @@
 namespace gegs {
 
 constexpr int PART_WORDS = 16;
+constexpr uint32_t PLAIN_BLOCK = 128;   // threads per block of the plain kernel
 
 struct StackSink {
     float *base;          // [slot][word][thread]
@@ -79,6 +80,12 @@ struct PlainArgs {
     Env env;
     const gegs_source *src;
     uint32_t first, last;        // source records [first, last)
+    // statistical batches of the run, equal slices of its n_run records from
+    // record run_first; this launch holds those from batch0 on, one dose row each
+    uint64_t run_first, n_run;
+    uint32_t n_batches, batch0;
+    size_t nvox;                 // length of a dose row
+    uint32_t lanes;              // lanes of a wavefront that take histories (plain_lanes)
     uint64_t hist_offset;        // global index of record 0
     uint32_t *next;              // work counter of this launch, starts at 0
     float *stack;
@@ -106,6 +113,20 @@ __device__ __forceinline__ Part source_particle(const gegs_source &r, int module
     return p;
 }
 
+// Lanes of a wavefront that take histories (or, in the event path's tail
+// launch, particles) when `n` of them are spread over `waves` resident
+// wavefronts.  The lanes of a wavefront follow different histories and take
+// their branches one after the other, so a full wavefront is the best for
+// throughput and the worst for the time of one history: while there are
+// fewer histories than resident lanes, each wavefront gets its share of them
+// and no more, which fills the chip with short wavefronts instead of a few
+// long ones (2 001 histories on 60^3 water: 3.6 ms in 32 full wavefronts,
+// 1.6 ms in 2 001 wavefronts of one lane).
+__host__ __device__ __forceinline__ uint32_t plain_lanes(uint64_t n, uint64_t waves) {
+    const uint64_t l = (n + waves - 1) / waves;
+    return (uint32_t)(l < 1 ? 1 : (l > 64 ? 64 : l));
+}
+
 template <bool TAB, bool GEN>
 __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) plain_kernel(PlainArgs a) {
     extern __shared__ float lds_env[];
@@ -125,10 +146,14 @@ __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) plain_kernel(PlainAr
 #pragma unroll
     for (int k = 0; k < N_EVENTS; ++k) pops[k] = 0;
     uint32_t nhist = 0;
-    for (;;) {
+    const bool takes = __lane_id() < a.lanes;
+    while (takes) {
         const uint32_t k = atomicAdd(a.next, 1u);
         if (k >= a.last - a.first) break;
         const uint32_t i = a.first + k;
+        // the batch of record off is the b-th slice [n b / nb, n (b + 1) / nb)
+        const uint64_t off = i - a.run_first;
+        t.dose = a.dose + (size_t)(((off + 1) * a.n_batches - 1) / a.n_run - a.batch0) * a.nvox;
         Part p = source_particle(a.src[i], env.fields[0].module_first);
         p.lin = primary_lineage(a.hist_offset + i);
         t.hist_edep = 0.0;
@@ -204,18 +229,6 @@ __global__ void sample_kernel(Env env, const gegs_particle *in, uint32_t n, gegs
     handle(env, s, p, sink, t);
     n_out[i] = sink.n;
     edep[i] = t.hist_edep;
-}
-
-// batch boundary: fold the batch tally into the run totals and clear it
-__global__ void fold_batch(double *chunk, double *dose, double *dose2, size_t n) {
-    for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x) {
-        const double d = chunk[v];
-        if (d != 0.0) {
-            dose[v] += d;
-            dose2[v] += d * d;
-            chunk[v] = 0.0;
-        }
-    }
 }
 
 // dose and dose2 of n_rows x nvox from nb per-batch rows each ([row][batch][voxel]),

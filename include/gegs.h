@@ -168,7 +168,8 @@ typedef struct gegs_tuning {
                                     the electron side concurrently, 1 = one after the other (2) */
     uint32_t tail_particles;     /* once every source record is injected and at most this many particles are in
                                     flight, one launch finishes them, each with its descendants in one thread
-                                    (262144, the most; 0xFFFFFFFF: never, the sweeps run to the end) */
+                                    (262144, the most; 0xFFFFFFFF: never, the sweeps run to the end); without
+                                    gegs_set_tuning a run of at most 8192 histories takes that launch at once */
     uint64_t capacity;           /* particles per bank, rounded down to a multiple of 32: each bank is 32 equal
                                     append segments, and a full segment counts as overflow (0: twice the
                                     injection plus the threshold, each at most the run's histories, and at
