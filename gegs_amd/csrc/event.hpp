@@ -571,8 +571,8 @@ struct HoldSink {
 // flights are appended together when the wavefront refills (or runs dry),
 // so that one atomic per destination serves many lanes.
 template <bool TAB, bool ADJ, bool GEN>
-__global__ void __launch_bounds__(512) photon_kernel(EvArgs a, uint32_t chunk, uint32_t refill_min,
-                                                     uint32_t refill_slots) {
+__global__ void __launch_bounds__(512) GEGS_WAVES_PER_EU(4) photon_kernel(EvArgs a, uint32_t chunk,
+                                                                          uint32_t refill_min, uint32_t refill_slots) {
     extern __shared__ float lds_env[];
     const uint32_t flip = a.st->flip;
     const int slot_in = bank_slot(P_PHOTON_STEP, flip, true);
@@ -582,7 +582,7 @@ __global__ void __launch_bounds__(512) photon_kernel(EvArgs a, uint32_t chunk, u
     if (Refill::block_share() >= n) return;   // no wavefront of the block has a share
     Env env = a.env;
     env.fixes = kernel_fixes<GEN>(env.fixes);
-    stage_env<TAB>(env, lds_env);
+    stage_env<TAB, TAB>(env, lds_env);
     TallyT<ADJ> t = fresh_tally<ADJ>(a);
     BankSink sink{&a, 0, flip, false, false};
     HoldSink hold{false};
@@ -603,6 +603,7 @@ __global__ void __launch_bounds__(512) photon_kernel(EvArgs a, uint32_t chunk, u
         const bool refills = !rf.empty() && (nidle >= refill_min || nidle == 64u);
         if (nheld && (refills || nheld >= refill_min || nidle == 64u)) {
             if (hold.held) {
+                photon_walk_leave(env, p, w);
                 // flights that reached their interaction point choose it now,
                 // together, from their untouched streams
                 if (interact) {
@@ -632,7 +633,7 @@ __global__ void __launch_bounds__(512) photon_kernel(EvArgs a, uint32_t chunk, u
                 have = false;
                 flush_particle(a, hist, t);
             } else {
-                const int r = photon_walk_iter(env, s, p, w, hold, t);
+                const int r = photon_walk_iter<TAB>(env, s, p, w, hold, t);
                 if (r != PW_ON) {
                     have = false;
                     flush_particle(a, hist, t);

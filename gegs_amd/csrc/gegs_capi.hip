@@ -29,6 +29,7 @@ struct gegs_ctx {
     uint16_t *d_rcls = nullptr;          // class index per region
     gegs_region *d_rtab = nullptr;       // distinct region records
     uint32_t nclass = 0;
+    bool odd_density = false;            // a density factor outside 2^-40 ... 2^40
     uint32_t max_med = 0;                // largest non-vacuum medium index of the phantom
     uint32_t nmed = 0;                   // media in the loaded tables
     float *d_xb = nullptr, *d_yb = nullptr, *d_zb = nullptr;
@@ -284,8 +285,13 @@ int gegs_load_phantom(gegs_ctx *c, uint32_t nx, uint32_t ny, uint32_t nz, const 
              "copy region table");
     c->nclass = (uint32_t)table.size();
     c->max_med = 0;
-    for (const gegs_region &r : table)
-        if (r.med != GEGS_VACUUM && r.med > c->max_med) c->max_med = r.med;
+    c->odd_density = false;
+    for (const gegs_region &r : table) {
+        if (r.med == GEGS_VACUUM) continue;
+        if (r.med > c->max_med) c->max_med = r.med;
+        // 2^-40 ... 2^40: quotients by the density stay normal (photon_walk_inner)
+        if (!(r.rhof >= 9.094947e-13f && r.rhof <= 1.0995116e12f)) c->odd_density = true;
+    }
     c->nx = nx;
     c->ny = ny;
     c->nz = nz;
@@ -580,7 +586,7 @@ static Env make_env(gegs_ctx *c, uint64_t seed, uint32_t njob) {
     env.jawx_next = c->have_mlc ? GEGS_M_MLC : env.mlc_next;
     env.bw = c->d_bw;
     env.wedge_nver = c->h_bw.wedge_nver;
-    env.fixes = c->fixes | c->media_opts;
+    env.fixes = c->fixes | c->media_opts | (c->odd_density ? ENV_ODD_DENSITY : 0u);
     env.seed = seed;
     return env;
 }

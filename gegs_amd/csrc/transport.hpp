@@ -120,7 +120,7 @@ struct Stream {
     uint32_t blk;            // block after the one being consumed
     int pos;                 // uniforms of the current block already used
     int nchild;
-    float b0, b1, b2, b3;    // current block
+    float b0, b1, b2, b3;    // uniforms of the current block still to use, the next one in b0
     float n0, n1, n2, n3;    // block blk, generated ahead of use when `ahead`
     bool ahead;
     uint32_t k0, k1;
@@ -170,12 +170,18 @@ struct Stream {
             blk -= 1;
             refill();
             pos = p.spos & 7;
+            if (pos & 1) { b0 = b1; b1 = b2; b2 = b3; }
+            if (pos & 2) { b0 = b2; b1 = b3; }
         }
     }
     __device__ __forceinline__ float next() {
         if (pos == 4) refill();
-        const int k = pos++;
-        return k == 0 ? b0 : (k == 1 ? b1 : (k == 2 ? b2 : b3));
+        pos++;
+        const float r = b0;
+        b0 = b1;
+        b1 = b2;
+        b2 = b3;
+        return r;
     }
     __device__ __forceinline__ uint64_t child() {
         const uint64_t at = (uint64_t)blk * 4u + (uint64_t)pos;
@@ -249,7 +255,9 @@ __host__ __device__ inline size_t env_lds_bytes(uint32_t nx, uint32_t ny, uint32
     return b;
 }
 
-template <bool TAB>
+// RCP: the staged region records hold 1 / rhof in place of ecut (photons do
+// not read ecut).
+template <bool TAB, bool RCP = false>
 __device__ __forceinline__ void stage_env(Env &env, float *lds) {
     float *p = lds;
     const gegs_region *rtab = env.rtab;
@@ -257,7 +265,11 @@ __device__ __forceinline__ void stage_env(Env &env, float *lds) {
     if (TAB) {
         float4 *rt = reinterpret_cast<float4 *>(p);
         const float4 *src = reinterpret_cast<const float4 *>(env.rtab);
-        for (uint32_t i = threadIdx.x; i < env.nclass; i += blockDim.x) rt[i] = src[i];
+        for (uint32_t i = threadIdx.x; i < env.nclass; i += blockDim.x) {
+            float4 rec = src[i];
+            if (RCP) rec.w = 1.0f / rec.y;     // gegs_region: med | flags, rhof, pcut, ecut
+            rt[i] = rec;
+        }
         rtab = reinterpret_cast<const gegs_region *>(rt);
         p += (size_t)env.nclass * 4;
         gegs_float2 *g = reinterpret_cast<gegs_float2 *>(p);
@@ -383,6 +395,9 @@ __device__ __forceinline__ Local phantom_frame64(const gegs_field &f, const Part
 // CUDA_EGS.h:35-38), set by the host from the tables.
 constexpr uint32_t ENV_PRESTA2 = 1u << 16;     // msdist_pII instead of msdist_pI
 constexpr uint32_t ENV_EXACT_BCA = 1u << 17;   // exact boundary crossing (single scattering)
+// a region record whose density factor is outside the range the photon walk's
+// reciprocal takes (set by the host from the phantom)
+constexpr uint32_t ENV_ODD_DENSITY = 1u << 18;
 constexpr uint32_t ENV_GENERAL = GEGS_FIX_FP64_FRAME | ENV_PRESTA2 | ENV_EXACT_BCA;
 
 // The flight and plain kernels are instantiated twice: GEN = false for the
@@ -641,7 +656,30 @@ struct PhotonWalk {
     float lu, lv, lw;        // direction in the phantom frame
     int32_t ix, iy, iz;      // voxel indices, valid when p.region >= VAC_AND_OTH
     float cohfac;            // Rayleigh factor of the last step (read by photon_interaction)
+    // state of the walk from voxel to voxel (inner), see photon_walk_inner
+    bool inner;              // p's position and direction are in the phantom's axis order
+    float fx, fy, fz;        // coordinate of the voxel face ahead on each axis
+    float yu, yv, yw;        // 1 / lu, 1 / lv, 1 / lw
+    float cosa, sina, isox, isoy, isoz, offy, offz;   // the field's frame
 };
+
+// by value: a ?: over two members would select their addresses and keep the
+// whole struct in memory
+template <class V>
+__device__ __forceinline__ V pick(bool c, V a, V b) { return c ? a : b; }
+
+// a / b correctly rounded, for y = 1 / b correctly rounded: the product is
+// within 1.5 ULP, the first correction within 1, and a corrected quotient
+// within 1 ULP rounds correctly after the second (Markstein 1990).  Needs the
+// remainders to be exact: |a| >= 2^-100 or 0, and no overflow.
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+constexpr float DIV_BY_MIN = 7.8886091e-31f;      // 2^-100
+constexpr float INNER_MIN_COS = 8.6736174e-19f;   // 2^-60: direction cosines the inner walk takes, or 0
+constexpr float FACE_NEVER = 1e30f;               // face ahead on an axis the flight is parallel to
 
 // photon_walk_iter's outcomes: the flight ended (absorbed below the cut,
 // discarded, or handed on), goes on, or reached its interaction point
@@ -681,7 +719,60 @@ __device__ __forceinline__ void decode_voxel(const Env &env, uint32_t region, in
     ix = (int32_t)(ir - (uint32_t)iy * env.nx);
 }
 
-__device__ __forceinline__ void photon_walk_begin(const Env &env, const Part &p, PhotonWalk &w) {
+// Starts the inner walk of a photon in a voxel that is not vacuum (nothing
+// happens for a direction cosine below 2^-60 or with the binary64 frame:
+// that flight stays with photon_walk_iter's general steps, as does one that
+// ends at its cuts).  The axis order
+// of the phantom (x, y, z or, with change_xyz, head y, z, x) is applied to
+// the position and the direction once: every step moves each coordinate by
+// its own cosine, whatever the order.
+__device__ __forceinline__ void photon_walk_enter(const Env &env, Part &p, PhotonWalk &w) {
+    const float au = fabsf(w.lu), av = fabsf(w.lv), aw = fabsf(w.lw);
+    const bool regular = (au == 0.0f || au >= INNER_MIN_COS) && (av == 0.0f || av >= INNER_MIN_COS) &&
+                         (aw == 0.0f || aw >= INNER_MIN_COS) && au < 2.0f && av < 2.0f && aw < 2.0f &&
+                         au + av + aw > 0.5f;
+    if (!regular || w.rd.med == VACUUM || p.e <= w.rd.pcut || p.wt <= 0.0f || (env.fixes & (GEGS_FIX_FP64_FRAME | ENV_ODD_DENSITY))) return;
+    const gegs_field &f = field_of(env, p);
+    w.cosa = f.cos_angle;
+    w.sina = f.sin_angle;
+    w.isox = f.iso_x;
+    w.isoy = f.iso_y;
+    w.isoz = f.iso_z;
+    w.offy = pick(f.change_xyz != 0, f.source_to_isocenter, 0.0f);
+    w.offz = pick(f.change_xyz != 0, 0.0f, f.source_to_isocenter);
+    if (f.change_xyz) {
+        const float x = p.x, u = p.u;
+        p.x = p.y; p.y = p.z; p.z = x;
+        p.u = p.v; p.v = p.w; p.w = u;
+    }
+    w.yu = au == 0.0f ? 1.0f : 1.0f / w.lu;
+    w.yv = av == 0.0f ? 1.0f : 1.0f / w.lv;
+    w.yw = aw == 0.0f ? 1.0f : 1.0f / w.lw;
+    w.fx = au == 0.0f ? FACE_NEVER : env.xb[w.ix + (w.lu > 0.0f ? 1 : 0)];
+    w.fy = av == 0.0f ? FACE_NEVER : env.yb[w.iy + (w.lv > 0.0f ? 1 : 0)];
+    w.fz = aw == 0.0f ? FACE_NEVER : env.zb[w.iz + (w.lw > 0.0f ? 1 : 0)];
+    // an axis parallel to the flight divides by 1: 1e30, beyond every other face
+    if (au == 0.0f) w.lu = 1.0f;
+    if (av == 0.0f) w.lv = 1.0f;
+    if (aw == 0.0f) w.lw = 1.0f;
+    w.inner = true;
+}
+
+// Ends the inner walk: position and direction back in the head's axis order.
+__device__ __forceinline__ void photon_walk_leave(const Env &env, Part &p, PhotonWalk &w) {
+    if (!w.inner) return;
+    w.inner = false;
+    if (w.fx == FACE_NEVER) w.lu = 0.0f;
+    if (w.fy == FACE_NEVER) w.lv = 0.0f;
+    if (w.fz == FACE_NEVER) w.lw = 0.0f;
+    if (field_of(env, p).change_xyz) {
+        const float x = p.x, u = p.u;
+        p.x = p.z; p.z = p.y; p.y = x;
+        p.u = p.w; p.w = p.v; p.v = u;
+    }
+}
+
+__device__ __forceinline__ void photon_walk_begin(const Env &env, Part &p, PhotonWalk &w) {
     w.rd = region_rec(env, p.region);
     w.gle = glog(p.e);
     w.cmed = -1;
@@ -692,16 +783,130 @@ __device__ __forceinline__ void photon_walk_begin(const Env &env, const Part &p,
     w.lv = q.v;
     w.lw = q.w;
     w.ix = w.iy = w.iz = 0;
-    if (p.region >= VAC_AND_OTH) decode_voxel(env, p.region, w.ix, w.iy, w.iz);
+    w.inner = false;
+    if (p.region >= VAC_AND_OTH) {
+        decode_voxel(env, p.region, w.ix, w.iy, w.iz);
+        photon_walk_enter(env, p, w);
+    }
+}
+
+// The free-flight segment of photon_walk_iter for a photon in a voxel of the
+// phantom that is not vacuum: the same values, in fewer instructions.
+//   * The frame, the face ahead on each axis and the reciprocals of the
+//     direction cosines stay in registers from crossing to crossing, so each
+//     face distance is a difference and a corrected product (div_by) instead
+//     of a division; the next face is read from LDS after a crossing.
+//   * RCP: the region table holds 1 / rhof in place of ecut, which photons
+//     do not read, and the mean free path takes div_by too.
+//   * Whether the path left over falls below EPSGMFP is decided from the
+//     distance left, which differs from the reference's
+//     dpmfp - tstep / gmfp by at most 4 x 2^-24 of dpmfp; only values closer
+//     than 16 x 2^-24 to the limit take that division.
+//   * The cuts are tested after the crossing only: the energy and the weight
+//     do not change in flight, and photon_walk_enter tested the first voxel.
+// Vector instructions bind the walk at full occupancy (86% issue on the
+// 128x128x100 CT, 488 lane slots a step before).  Measured: event loop 1e7
+// histories 42.8 -> 36.9 ms, plain kernel 1e6 35.3 -> 26.0 ms, 20 011 on 60^3
+// water without allocation 2.7 -> 1.7 ms.  The event loop's photon kernel
+// holds 4 waves per SIMD (128 VGPRs, 2 spilled; 133 without the limit, 3
+// waves and 40.0 ms).
+template <bool RCP, class Sink, class T>
+__device__ __forceinline__ int photon_walk_inner(const Env &env, Stream &s, Part &p, PhotonWalk &w, Sink &sink, T &t) {
+    t.photon_steps++;
+    t.steps++;
+    const gegs_region rd0 = w.rd;
+    const float y = p.y - w.offy, z = p.z - w.offz;
+    const float rx = p.x * w.cosa - y * w.sina;
+    const float ry = p.x * w.sina + y * w.cosa;
+    const float ax = w.fx - (rx + w.isox), ay = w.fy - (ry + w.isoy), az = w.fz - (z + w.isoz);
+    float dx = div_by(ax, w.lu, w.yu), dy = div_by(ay, w.lv, w.yv), dz = div_by(az, w.lw, w.yw);
+    if (fminf(fminf(fabsf(ax), fabsf(ay)), fabsf(az)) < DIV_BY_MIN) {
+        dx = ax / w.lu;
+        dy = ay / w.lv;
+        dz = az / w.lw;
+    }
+    // the last face of minimal distance, in x, y, z order
+    const bool y_le = dy <= dx;
+    float dmin = y_le ? dy : dx;
+    const bool z_le = dz <= dmin;
+    dmin = z_le ? dz : dmin;
+    const uint32_t nx = env.nx, ny = env.ny;
+    const bool up = pick(z_le, w.lw, pick(y_le, w.lv, w.lu)) > 0.0f;
+    const int32_t inew = pick(z_le, w.iz, pick(y_le, w.iy, w.ix)) + (up ? 1 : -1);
+    const uint32_t nsel = pick(z_le, env.nz, pick(y_le, ny, nx));
+    const int32_t stride = pick(z_le, (int32_t)(nx * ny), pick(y_le, (int32_t)nx, 1));
+    const uint32_t ncand = (uint32_t)inew < nsel ? p.region + (uint32_t)(up ? stride : -stride) : 0u;
+    const uint16_t cls_next = env.rcls[ncand];
+    const float r1 = s.next();
+    const float dpmfp = -glog_normal(r1);
+    if ((int32_t)rd0.med != w.cmed) {
+        const gegs_float2 ge = env.pge[rd0.med];
+        w.lgle = (int)(ge.x + ge.y * w.gle);
+        const gegs_float2 gm = env.pgmfp[rd0.med * MXGE + w.lgle];
+        const gegs_float2 ch = env.pcohe[rd0.med * MXGE + w.lgle];
+        w.gmfpr0 = gm.x + gm.y * w.gle;
+        w.cohf = ch.x + ch.y * w.gle;
+        w.cmed = rd0.med;
+    }
+    float gmfp_val;
+    if (RCP && fabsf(w.gmfpr0) >= INNER_MIN_COS) gmfp_val = div_by(w.gmfpr0, rd0.rhof, rd0.ecut);
+    else gmfp_val = w.gmfpr0 / rd0.rhof;
+    float cohfac = 0.0f;
+    if (rd0.flags & GEGS_F_RAYLEIGH) {
+        cohfac = w.cohf;
+        gmfp_val *= cohfac;
+    }
+    const float path = gmfp_val * dpmfp;
+    const bool crossed = dmin <= path;
+    float tstep = crossed ? dmin : path;
+    if (tstep < 0.0f) tstep = EPSTEP;
+    int idisc = 0;
+    if (crossed && ncand == 0) {
+        if (p.leaf == PASSMLC) {
+            p.region = 0;
+            return PW_END;
+        }
+        idisc = -1;
+    }
+    p.x += p.u * tstep;
+    p.y += p.v * tstep;
+    p.z += p.w * tstep;
+    if (crossed) {
+        // the axis crossed gets its next face
+        const int32_t at = pick(z_le, (int32_t)(env.zb - env.xb), pick(y_le, (int32_t)(env.yb - env.xb), 0));
+        const float face = env.xb[at + inew + (up ? 1 : 0)];
+        const bool x_sel = !z_le && !y_le, y_sel = !z_le && y_le;
+        w.fx = pick(x_sel, face, w.fx);
+        w.fy = pick(y_sel, face, w.fy);
+        w.fz = pick(z_le, face, w.fz);
+        w.ix = pick(x_sel, inew, w.ix);
+        w.iy = pick(y_sel, inew, w.iy);
+        w.iz = pick(z_le, inew, w.iz);
+        w.rd = env.rtab[cls_next];
+        p.region = ncand;
+        t.gathers++;
+    }
+    if (p.e <= w.rd.pcut || idisc < 0) { t.score(p.region, p.e * p.wt); return PW_END; }
+    if (w.rd.med != rd0.med) {
+        if (w.rd.med == VACUUM) photon_walk_leave(env, p, w);
+        return PW_ON;
+    }
+    const float left = path - tstep, slack = 1e-6f * dpmfp;
+    if (left > gmfp_val * (1e-5f + slack)) return PW_ON;
+    if (!(left < gmfp_val * (1e-5f - slack)) &&
+        (double)fmaxf(0.0f, dpmfp - tstep / gmfp_val) >= EPSGMFP) return PW_ON;
+    w.cohfac = cohfac;
+    return PW_INTERACT;
 }
 
 // One free-flight segment: PW_ON when the photon crossed a boundary and flies
 // on, PW_INTERACT at the interaction point (photon_interaction then chooses
 // the interaction from the same stream; the event path defers that choice
 // until the wavefront hands its ended flights on together), PW_END otherwise.
-template <class Sink, class T>
+// RCP: see photon_walk_inner.
+template <bool RCP = false, class Sink, class T>
 __device__ __forceinline__ int photon_walk_iter(const Env &env, Stream &s, Part &p, PhotonWalk &w, Sink &sink, T &t) {
-    const gegs_media_tables *mt = env.mt;
+    if (w.inner) return photon_walk_inner<RCP>(env, s, p, w, sink, t);
     t.photon_steps++;
     t.steps++;
     gegs_region rd = w.rd;
@@ -814,7 +1019,10 @@ __device__ __forceinline__ int photon_walk_iter(const Env &env, Stream &s, Part 
         t.gathers++;
     }
     if (p.e <= rd.pcut || idisc < 0) { t.score(p.region, p.e * p.wt); return PW_END; }
-    if (rd.med != old_med || rd.med == VACUUM || (double)dpmfp >= EPSGMFP) return PW_ON;
+    if (rd.med != old_med || rd.med == VACUUM || (double)dpmfp >= EPSGMFP) {
+        if (p.region >= VAC_AND_OTH) photon_walk_enter(env, p, w);
+        return PW_ON;
+    }
     // the interaction point: the medium is the one the step started in, so
     // w.lgle and w.gle index its rows; the Rayleigh factor is the step's
     w.cohfac = cohfac;
@@ -867,6 +1075,7 @@ __device__ __forceinline__ void photon_step(const Env &env, Stream &s, Part &p, 
         if (VOTE) wave_lookahead(s, true);
         const int r = photon_walk_iter(env, s, p, w, sink, t);
         if (r == PW_ON) continue;
+        photon_walk_leave(env, p, w);
         if (r == PW_INTERACT) photon_interaction(env, s, p, w, sink);
         break;
     }

@@ -21,3 +21,14 @@ def test_polygon_tests_equal_their_plain_forms(tmp_path):
     r = subprocess.run([exe, "6000"], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]
     assert r.stdout.startswith("checks 2400000")
+
+
+def test_walk_quotients_and_logarithm_equal_their_plain_forms(tmp_path):
+    """div_by against the division for the operands the photon walk gives it,
+    and glog against its form with the exponent and mantissa taken apart."""
+    exe = str(tmp_path / "walk_check")
+    subprocess.check_call([CLANG, "-std=c++17", "-O2", "-mfma", "-ffp-contract=off", "-I",
+                           os.path.join(HERE, "cpu_event", "include"), "-DLDS_FLOATS=1", "-o", exe,
+                           os.path.join(HERE, "cpu_event", "walk_check.cpp")])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr[-2000:]
