@@ -873,8 +873,9 @@ __device__ __forceinline__ int photon_walk_inner(const Env &env, Stream &s, Part
     p.z += p.w * tstep;
     if (crossed) {
         // the axis crossed gets its next face
-        const int32_t at = pick(z_le, (int32_t)(env.zb - env.xb), pick(y_le, (int32_t)(env.yb - env.xb), 0));
-        const float face = env.xb[at + inew + (up ? 1 : 0)];
+        const float *bounds = pick(z_le, env.zb, pick(y_le, env.yb, env.xb));
+        const int32_t at = inew + (up ? 1 : 0);
+        const float face = bounds[at < 0 ? 0 : at];   // left through the lowest face: no next one, the flight ends
         const bool x_sel = !z_le && !y_le, y_sel = !z_le && y_le;
         w.fx = pick(x_sel, face, w.fx);
         w.fy = pick(y_sel, face, w.fy);

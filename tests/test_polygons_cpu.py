@@ -32,3 +32,16 @@ def test_walk_quotients_and_logarithm_equal_their_plain_forms(tmp_path):
                            os.path.join(HERE, "cpu_event", "walk_check.cpp")])
     r = subprocess.run([exe], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr[-2000:]
+
+
+def test_walk_takes_each_axis_bounds_from_its_own_array(tmp_path):
+    """Kernels that stage nothing in LDS have the three bounds in allocations
+    of their own, any distance apart; and a flight that leaves through the
+    lowest face of an axis reads nothing before them (address checks on)."""
+    exe = str(tmp_path / "walk_bounds_check")
+    subprocess.check_call([CLANG, "-std=c++17", "-O1", "-g", "-fsanitize=address", "-fno-omit-frame-pointer",
+                           "-ffp-contract=off", "-I", os.path.join(HERE, "cpu_event", "include"), "-DLDS_FLOATS=1",
+                           "-o", exe, os.path.join(HERE, "cpu_event", "walk_bounds_check.cpp")])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120,
+                       env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout, r.stderr[-2000:])
