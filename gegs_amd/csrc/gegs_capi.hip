@@ -768,11 +768,13 @@ int gegs_run_plain_noalloc(gegs_ctx *c, const gegs_run_options *o, double *dose,
     const uint32_t block = o->block_size ? o->block_size : PLAIN_BLOCK;
     if (block != PLAIN_BLOCK) return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: block_size must be 128");
     const int depth = o->stack_depth ? (int)o->stack_depth : 40;
-    // an explicit grid keeps the room for stacks that one row leaves
-    const uint32_t rows = o->grid_size ? 1u : batch_rows(NOALLOC_ROW_BYTES, c->nvox, o->n_batches);
-    const NoallocLayout L(c->nvox, rows);
     const size_t per_block = (size_t)block * depth * PART_WORDS * sizeof(float);
     const size_t cap = GEGS_NOALLOC_SCRATCH_BYTES;
+    // an explicit grid, or stacks so deep that a block needs it, keeps the
+    // room for stacks that one row leaves
+    uint32_t rows = o->grid_size ? 1u : batch_rows(NOALLOC_ROW_BYTES, c->nvox, o->n_batches);
+    if (NoallocLayout(c->nvox, rows).stack + per_block > cap) rows = 1;
+    const NoallocLayout L(c->nvox, rows);
     if (L.stack + per_block > cap)
         return fail(c, GEGS_ERR_ARG, "run_plain_noalloc: the phantom's dose row and one block of particle stacks "
                                      "exceed the scratch size (GEGS_NOALLOC_SCRATCH_BYTES)");

@@ -60,3 +60,21 @@ def test_noalloc_batches_in_several_launches(gpu_ctx, n, n_batches):
     assert c["photon_steps"] == p["counters"]["photon_steps"]
     assert np.allclose(dose.cpu().numpy(), p["dose"], rtol=1e-13, atol=1e-13)
     assert np.allclose(dose2.cpu().numpy(), p["dose2"], rtol=1e-13, atol=1e-13)
+
+
+def test_noalloc_deep_stacks_keep_their_room(gpu_ctx):
+    """One block of stacks 28 000 deep takes 229 MB of the 256 MiB scratch: it
+    fits beside one dose row of the CT, as before, not beside five."""
+    import torch
+    print("short runs: no-alloc, deep stacks", flush=True)
+    ctx = gpu_ctx
+    wl = workloads.ct()
+    ctx.load_workload(wl)
+    ctx.set_source(wl.source(100, 17))
+    p = ctx.run(seed=29, n_batches=5, method="plain")
+    dose = torch.empty(ctx.nvox, dtype=torch.float64, device="cuda")
+    dose2 = torch.empty_like(dose)
+    torch.cuda.synchronize()
+    c = ctx.run_plain_noalloc(29, dose.data_ptr(), dose2.data_ptr(), n_batches=5, depth=28000)
+    assert c["histories"] == 100 and c["overflow"] == 0
+    assert np.allclose(dose.cpu().numpy(), p["dose"], rtol=1e-13, atol=1e-13)
