@@ -97,8 +97,27 @@ struct EventConfig {
     uint32_t inject = 6u << 20;      // primaries injected per refill
     uint32_t threshold = 6u << 20;   // refill when fewer particles are in flight
     uint32_t sweeps_per_graph = 4;
+    bool pick_shape = true;          // chunks and grid by the run's fields (pick_shape), not the three above
     bool direct = true;              // a run of at most TAIL_DIRECT histories takes the tail launch at once
 };
+
+// Chunks and interaction blocks of a run whose caller gave none of the three.
+// A chunk costs its particles a bank round trip and bounds the sweep by its
+// slowest wavefront: crossings from voxel to voxel are cheap (about 1/8 of a
+// crossing in the MLC or of a condensed-history step), so photons go far per
+// sweep where every field starts in the phantom, while the long electron
+// chains of the head's tungsten keep theirs short; 512 blocks of the
+// interaction kernels leave room for the flights beside them.  Run times (ms)
+// at 32/16 with 2048 blocks and at 96/12 with 512: CT 1e7 37.1, 33.2; water 1e6
+// 7.1, 6.2; CT 3e5 with PRESTA-II 9.9, 8.0; gradient 4e6 39.1, 33.2; three
+// plans on 256x256x180 42.4, 36.5.  The 5-field MLC plan of 2e6: 32/16 59.1,
+// 32/8 55.7, 96/12 60.0.
+inline void pick_shape(EventConfig &cfg, bool head) {
+    if (!cfg.pick_shape) return;
+    cfg.photon_chunk = head ? 32 : 96;
+    cfg.electron_chunk = head ? 8 : 12;
+    cfg.grid = 512;
+}
 
 // Source records of one batch, as slices of every job (field) of the run:
 // cursor k of the batch belongs to job j with prefix[j] <= k < prefix[j+1];

@@ -883,7 +883,10 @@ static int run_event_jobs(gegs_ctx *c, const gegs_run_options *o, const std::vec
     }
     rc = upload_jobs(c, fields, plans, sets);
     if (rc) return rc;
-    const EventConfig cfg = c->tuning;
+    EventConfig cfg = c->tuning;
+    bool head = false;
+    for (const gegs_field &f : fields) head |= f.module_first != GEGS_M_PHANTOM;
+    pick_shape(cfg, head);
     Env env = make_env(c, o->seed, (uint32_t)jobs.size());
     hipError_t e = c->banks.reserve(total_all, nb, cfg);
     if (e != hipSuccess) return fail(c, GEGS_ERR_DEVICE, "event banks", e);
@@ -1067,6 +1070,7 @@ int gegs_set_tuning(gegs_ctx *c, const gegs_tuning *t) {
     EventConfig cfg;
     if (t) {
         cfg.direct = false;   // a caller's shape of the sweeps holds for runs of any length
+        cfg.pick_shape = !t->photon_chunk && !t->electron_chunk && !t->grid;
         if (t->block) cfg.block = t->block;
         if (t->flight_block) cfg.flight_block = t->flight_block;
         if (t->refill_min) cfg.refill_min = t->refill_min;

@@ -153,7 +153,8 @@ typedef struct gegs_run_options {
  * autotuner (gegs_amd/autotune.py) picks them per workload. */
 typedef struct gegs_tuning {
     uint32_t block;              /* threads per block of the single-pass event kernels: 64, 128 or 256 (256) */
-    uint32_t grid;               /* blocks of the single-pass event kernels (2048) */
+    uint32_t grid;               /* blocks of the single-pass event kernels (2048; with no grid and no
+                                    chunk given a run picks the three by its fields) */
     uint32_t photon_grid;        /* blocks of the photon kernel (enough to fill every CU once) */
     uint32_t electron_grid;      /* blocks of the electron kernel (same) */
     uint32_t photon_chunk;       /* voxel crossings per photon and sweep (32; 0xFFFFFFFF: no limit) */
