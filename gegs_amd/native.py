@@ -357,8 +357,8 @@ class Context:
         arr = self._jobs(jobs)
         self._check(self.L.gegs_set_history_tally(self.h, 1 if per_history else 0))
         opt = RunOptions(seed, 0, n_batches, 0, 0, 0, 0, 0)
-        dose = np.zeros(n_plans * self.nvox, dtype=np.float64)
-        dose2 = np.zeros(n_plans * self.nvox, dtype=np.float64)
+        dose = np.empty(n_plans * self.nvox, dtype=np.float64)      # written whole by the call
+        dose2 = np.empty(n_plans * self.nvox, dtype=np.float64)
         self._check(self.L.gegs_run_batched(self.h, arr, len(jobs), n_plans, ctypes.byref(opt), _p(dose), _p(dose2)))
         out = dict(dose=dose.reshape(n_plans, self.nvox), dose2=dose2.reshape(n_plans, self.nvox), n_batches=n_batches)
         ms = ctypes.c_float()
@@ -410,8 +410,8 @@ class Context:
             grid=0, block=0, depth=0, first=0, count=0):
         self._check(self.L.gegs_set_history_tally(self.h, 1 if per_history else 0))
         opt = RunOptions(seed, history_offset, n_batches, block, grid, depth, first, count)
-        dose = np.zeros(self.nvox, dtype=np.float64)
-        dose2 = np.zeros(self.nvox, dtype=np.float64)
+        dose = np.empty(self.nvox, dtype=np.float64)      # written whole by the call
+        dose2 = np.empty(self.nvox, dtype=np.float64)
         fn = self.L.gegs_run_plain if method == "plain" else self.L.gegs_run_event
         self._check(fn(self.h, ctypes.c_void_p(ctypes.addressof(opt)), _p(dose), _p(dose2)))
         out = dict(dose=dose, dose2=dose2, n_batches=n_batches)
