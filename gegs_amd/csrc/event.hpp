@@ -826,8 +826,8 @@ __global__ void sweep_end(EvState *st, uint32_t threshold, uint32_t max_inject) 
 // suspended electron resumes from its banked step state.  It is bound by the
 // longest chain of dependent steps of one wavefront, so the particles are
 // spread over all resident wavefronts, a few lanes of each (plain_lanes):
-// 1 000 histories' last particles on the CT 1.71 -> 1.1 ms, 100 003 through
-// jaws and MLC 17.9 -> 12 ms against 64 lanes each.
+// against 64 lanes each, a run's kernels went from 3.85 to 2.63 ms at 1 000
+// histories on the CT and from 27.5 to 22.3 ms at 100 003 through jaws and MLC.
 template <bool TAB, bool ADJ, bool GEN>
 __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) tail_kernel(EvArgs a, float *stack, int depth,
                                                                         uint32_t waves) {
