@@ -11,7 +11,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -19,12 +18,9 @@
 #include "ctimport.hpp"
 #include "event.hpp"
 #include "plain.hpp"
+#include "readback.hpp"
 
 using namespace gegs;
-
-// Pinned staging of read_back: 8 MiB per context.
-static constexpr int STAGE_SLOTS = 8;
-static constexpr size_t STAGE_BYTES = (size_t)1 << 20;
 
 struct gegs_ctx {
     int device = 0;
@@ -82,8 +78,7 @@ struct gegs_ctx {
     uint64_t hist_n = 0;
     gegs_counters counters{};
     float last_ms = 0.0f;
-    unsigned char *h_stage = nullptr;    // pinned slots of read_back
-    hipEvent_t stage_done[STAGE_SLOTS] = {};
+    ReadStage stage;                     // pinned slots of read_back
     EventBanks banks;
     EventConfig tuning;
     hipError_t scratch_err = hipSuccess; // address of this device's no-alloc scratch
@@ -198,9 +193,7 @@ void gegs_destroy(gegs_ctx *c) {
     hipFree(c->d_bweight);
     hipFree(c->d_adj);
     hipFree(c->d_grad);
-    if (c->h_stage) hipHostFree(c->h_stage);
-    for (int k = 0; k < STAGE_SLOTS; ++k)
-        if (c->stage_done[k]) hipEventDestroy(c->stage_done[k]);
+    c->stage.release();
     c->banks.release();
     hipStreamDestroy(c->stream);
     delete c;
@@ -601,63 +594,6 @@ static Env make_env(gegs_ctx *c, uint64_t seed, uint32_t njob) {
     return env;
 }
 
-// Device memory into the caller's pageable buffers.  A copy of a dose spends
-// most of its time on the host: the transfer into pinned memory runs at the
-// link's rate, while moving it on into pages that the caller never touched
-// is bound by one core.  Here up to STAGE_SLOTS host threads take the pieces
-// in turn, each through its own pinned slot, so the transfers of some pieces
-// run beside the host copies of the others (two doses of 13 MB on the
-// 128x128x100 CT: 1.9 -> 1.2 ms of a run).  Small results take a plain copy.  The
-// context's work must be complete.
-static hipError_t read_back(gegs_ctx *c, void *const *dst, const void *const *src, int n, size_t bytes) {
-    const size_t pieces = (bytes + STAGE_BYTES - 1) / STAGE_BYTES;
-    const size_t total = pieces * (size_t)n;
-    if (total >= 2 && !c->h_stage) {
-        hipError_t e = hipHostMalloc(&c->h_stage, STAGE_SLOTS * STAGE_BYTES);
-        if (e != hipSuccess) {
-            c->h_stage = nullptr;
-            return e;
-        }
-        for (int k = 0; k < STAGE_SLOTS; ++k)
-            if ((e = hipEventCreateWithFlags(&c->stage_done[k], hipEventDisableTiming)) != hipSuccess) return e;
-    }
-    if (total < 2) {
-        for (int k = 0; k < n; ++k) {
-            const hipError_t e = hipMemcpy(dst[k], src[k], bytes, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
-    hipError_t err[STAGE_SLOTS] = {};
-    auto work = [&](int slot) {
-        hipError_t e = hipSetDevice(c->device);
-        for (size_t i = (size_t)slot; i < total && e == hipSuccess; i += STAGE_SLOTS) {
-            const size_t at = i % pieces * STAGE_BYTES, len = bytes - at < STAGE_BYTES ? bytes - at : STAGE_BYTES;
-            unsigned char *stage = c->h_stage + slot * STAGE_BYTES;
-            e = hipMemcpyAsync(stage, (const unsigned char *)src[i / pieces] + at, len, hipMemcpyDeviceToHost, c->stream);
-            if (e == hipSuccess) e = hipEventRecord(c->stage_done[slot], c->stream);
-            if (e == hipSuccess) e = hipEventSynchronize(c->stage_done[slot]);
-            if (e == hipSuccess) memcpy((unsigned char *)dst[i / pieces] + at, stage, len);
-        }
-        err[slot] = e;
-    };
-    std::thread helper[STAGE_SLOTS - 1];
-    int started = 0;
-    try {
-        while (started < STAGE_SLOTS - 1 && (size_t)(started + 1) < total) {
-            helper[started] = std::thread(work, started + 1);
-            ++started;
-        }
-    } catch (...) {   // no thread to be had: this one takes the slots left
-    }
-    work(0);
-    for (int k = started + 1; k < STAGE_SLOTS; ++k) work(k);
-    for (int k = 0; k < started; ++k) helper[k].join();
-    for (int k = 0; k < STAGE_SLOTS; ++k)
-        if (err[k] != hipSuccess) return err[k];
-    return hipSuccess;
-}
-
 // dose and dose2 are host buffers, or device buffers with dev_out
 static int finish_run(gegs_ctx *c, double *dose, double *dose2, hipEvent_t t0, hipEvent_t t1, uint32_t n_plans = 1,
                       bool dev_out = false) {
@@ -689,7 +625,7 @@ static int finish_run(gegs_ctx *c, double *dose, double *dose2, hipEvent_t t0, h
         int k = 0;
         if (dose) { dst[k] = dose; src[k++] = c->d_dose; }
         if (dose2) { dst[k] = dose2; src[k++] = c->d_dose2; }
-        HIPCHECK(c, read_back(c, dst, src, k, n * sizeof(double)), "read dose");
+        HIPCHECK(c, read_back(c->stage, c->device, c->stream, dst, src, k, n * sizeof(double)), "read dose");
     }
     if (c->counters.overflow) return fail(c, GEGS_ERR_QUEUE_OVERFLOW, "particle stack overflow: particles were lost");
     return GEGS_OK;
