@@ -40,6 +40,7 @@
 #ifndef GEGS_WAVE_SUBSET_OP
 #define GEGS_WAVE_SUBSET_OP(id)
 #endif
+#include <cstring>
 #include <vector>
 
 #include "plain.hpp"
@@ -84,11 +85,11 @@ struct EvState {
 struct EventConfig {
     uint32_t block = 256;            // threads per block of the single-pass event kernels (<= 256)
     uint32_t flight_block = 256;     // threads per block of the photon and electron kernels (<= 512)
-    uint32_t grid = 2048;            // blocks of the single-pass interaction kernels
+    uint32_t grid = 0;               // blocks of the single-pass interaction kernels (0: by the run's fields)
     uint32_t photon_grid = 0;        // blocks of the photon kernel (0: fill the device once)
     uint32_t electron_grid = 0;      // blocks of the electron kernel (0: fill the device once)
-    uint32_t photon_chunk = 32;      // voxel crossings per photon and sweep (0: whole flight)
-    uint32_t electron_chunk = 16;    // condensed-history steps per electron and sweep (0: no limit)
+    uint32_t photon_chunk = 0;       // voxel crossings per photon and sweep (0: by the run's fields)
+    uint32_t electron_chunk = 0;     // condensed-history steps per electron and sweep (0: by the run's fields)
     uint32_t refill_min = 16;        // idle lanes of a wavefront that trigger a refill
     uint32_t refill_slots = 64;      // bank slots a wavefront reserves per refill atomic
     uint32_t sweep_streams = 2;      // 2: photon and electron sides of a sweep concurrently; 1: one after the other
@@ -97,11 +98,56 @@ struct EventConfig {
     uint32_t inject = 6u << 20;      // primaries injected per refill
     uint32_t threshold = 6u << 20;   // refill when fewer particles are in flight
     uint32_t sweeps_per_graph = 4;
-    bool pick_shape = true;          // chunks and grid by the run's fields (pick_shape), not the three above
     bool direct = true;              // a run of at most TAIL_DIRECT histories takes the tail launch at once
 };
 
-// Chunks and interaction blocks of a run whose caller gave none of the three.
+// The caller's tuning over the defaults (a zero field takes its default) and
+// back: what is left to the run is reported as 0, so that a tuning that was
+// read and set again changes nothing.
+inline gegs_tuning tuning_of(const EventConfig &cfg) {
+    gegs_tuning t{};
+    t.block = cfg.block;
+    t.grid = cfg.grid;
+    t.photon_grid = cfg.photon_grid;
+    t.electron_grid = cfg.electron_grid;
+    t.photon_chunk = cfg.photon_chunk;
+    t.electron_chunk = cfg.electron_chunk;
+    t.inject = cfg.inject;
+    t.threshold = cfg.threshold;
+    t.sweeps_per_graph = cfg.sweeps_per_graph;
+    t.flight_block = cfg.flight_block;
+    t.refill_min = cfg.refill_min;
+    t.refill_slots = cfg.refill_slots;
+    t.sweep_streams = cfg.sweep_streams;
+    t.tail_particles = cfg.tail ? cfg.tail : 0xFFFFFFFFu;
+    t.capacity = cfg.capacity;
+    return t;
+}
+
+inline EventConfig config_of(const gegs_tuning &t) {
+    EventConfig cfg;
+    if (t.block) cfg.block = t.block;
+    if (t.flight_block) cfg.flight_block = t.flight_block;
+    if (t.refill_min) cfg.refill_min = t.refill_min;
+    cfg.grid = t.grid;
+    cfg.photon_grid = t.photon_grid;
+    cfg.electron_grid = t.electron_grid;
+    cfg.photon_chunk = t.photon_chunk;
+    cfg.electron_chunk = t.electron_chunk;
+    if (t.inject) cfg.inject = t.inject;
+    if (t.threshold) cfg.threshold = t.threshold;
+    if (t.sweeps_per_graph) cfg.sweeps_per_graph = t.sweeps_per_graph;
+    cfg.capacity = (size_t)t.capacity;
+    if (t.refill_slots) cfg.refill_slots = t.refill_slots;
+    if (t.sweep_streams) cfg.sweep_streams = t.sweep_streams;
+    if (t.tail_particles) cfg.tail = t.tail_particles == 0xFFFFFFFFu ? 0u : t.tail_particles;
+    // a caller's shape of the sweeps holds for runs of any length
+    const gegs_tuning mine = tuning_of(cfg), dflt = tuning_of(EventConfig());
+    cfg.direct = memcmp(&mine, &dflt, sizeof(gegs_tuning)) == 0;
+    return cfg;
+}
+
+// Chunks and interaction blocks of a run, as far as its caller gave none.
 // A chunk costs its particles a bank round trip and bounds the sweep by its
 // slowest wavefront: crossings from voxel to voxel are cheap (about 1/8 of a
 // crossing in the MLC or of a condensed-history step), so photons go far per
@@ -113,10 +159,9 @@ struct EventConfig {
 // plans on 256x256x180 42.4, 36.5.  The 5-field MLC plan of 2e6: 32/16 59.1,
 // 32/8 55.7, 96/12 60.0.
 inline void pick_shape(EventConfig &cfg, bool head) {
-    if (!cfg.pick_shape) return;
-    cfg.photon_chunk = head ? 32 : 96;
-    cfg.electron_chunk = head ? 8 : 12;
-    cfg.grid = 512;
+    if (!cfg.photon_chunk) cfg.photon_chunk = head ? 32 : 96;
+    if (!cfg.electron_chunk) cfg.electron_chunk = head ? 8 : 12;
+    if (!cfg.grid) cfg.grid = 512;
 }
 
 // Source records of one batch, as slices of every job (field) of the run:

@@ -1074,26 +1074,7 @@ int gegs_set_beamlet_weights_device(gegs_ctx *c, const float *weight, uint32_t n
 
 int gegs_set_tuning(gegs_ctx *c, const gegs_tuning *t) {
     if (!c) return GEGS_ERR_ARG;
-    EventConfig cfg;
-    if (t) {
-        cfg.direct = false;   // a caller's shape of the sweeps holds for runs of any length
-        cfg.pick_shape = !t->photon_chunk && !t->electron_chunk && !t->grid;
-        if (t->block) cfg.block = t->block;
-        if (t->flight_block) cfg.flight_block = t->flight_block;
-        if (t->refill_min) cfg.refill_min = t->refill_min;
-        if (t->grid) cfg.grid = t->grid;
-        cfg.photon_grid = t->photon_grid;
-        cfg.electron_grid = t->electron_grid;
-        if (t->photon_chunk) cfg.photon_chunk = t->photon_chunk;
-        if (t->electron_chunk) cfg.electron_chunk = t->electron_chunk;
-        if (t->inject) cfg.inject = t->inject;
-        if (t->threshold) cfg.threshold = t->threshold;
-        if (t->sweeps_per_graph) cfg.sweeps_per_graph = t->sweeps_per_graph;
-        if (t->capacity) cfg.capacity = (size_t)t->capacity;
-        if (t->refill_slots) cfg.refill_slots = t->refill_slots;
-        if (t->sweep_streams) cfg.sweep_streams = t->sweep_streams;
-        if (t->tail_particles) cfg.tail = t->tail_particles == 0xFFFFFFFFu ? 0u : t->tail_particles;
-    }
+    const EventConfig cfg = t ? config_of(*t) : EventConfig();
     if (cfg.tail > (1u << 18)) return fail(c, GEGS_ERR_ARG, "gegs_set_tuning: tail_particles above 262144");
     if (cfg.sweep_streams != 1 && cfg.sweep_streams != 2)
         return fail(c, GEGS_ERR_ARG, "gegs_set_tuning: sweep_streams must be 1 or 2");
@@ -1116,22 +1097,7 @@ int gegs_set_tuning(gegs_ctx *c, const gegs_tuning *t) {
 
 int gegs_get_tuning(gegs_ctx *c, gegs_tuning *t) {
     if (!c || !t) return GEGS_ERR_ARG;
-    const EventConfig &cfg = c->tuning;
-    t->block = cfg.block;
-    t->grid = cfg.grid;
-    t->photon_grid = cfg.photon_grid;
-    t->electron_grid = cfg.electron_grid;
-    t->photon_chunk = cfg.photon_chunk;
-    t->electron_chunk = cfg.electron_chunk;
-    t->inject = cfg.inject;
-    t->threshold = cfg.threshold;
-    t->sweeps_per_graph = cfg.sweeps_per_graph;
-    t->flight_block = cfg.flight_block;
-    t->refill_min = cfg.refill_min;
-    t->refill_slots = cfg.refill_slots;
-    t->sweep_streams = cfg.sweep_streams;
-    t->tail_particles = cfg.tail ? cfg.tail : 0xFFFFFFFFu;
-    t->capacity = cfg.capacity;
+    *t = tuning_of(c->tuning);
     return GEGS_OK;
 }
 

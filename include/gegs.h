@@ -153,12 +153,13 @@ typedef struct gegs_run_options {
  * autotuner (gegs_amd/autotune.py) picks them per workload. */
 typedef struct gegs_tuning {
     uint32_t block;              /* threads per block of the single-pass event kernels: 64, 128 or 256 (256) */
-    uint32_t grid;               /* blocks of the single-pass event kernels (2048; with no grid and no
-                                    chunk given a run picks the three by its fields) */
+    uint32_t grid;               /* blocks of the single-pass event kernels (picked by the run: 512) */
     uint32_t photon_grid;        /* blocks of the photon kernel (enough to fill every CU once) */
     uint32_t electron_grid;      /* blocks of the electron kernel (same) */
-    uint32_t photon_chunk;       /* voxel crossings per photon and sweep (32; 0xFFFFFFFF: no limit) */
-    uint32_t electron_chunk;     /* condensed-history steps per electron and sweep (16; 0xFFFFFFFF: no limit) */
+    uint32_t photon_chunk;       /* voxel crossings per photon and sweep (picked by the run: 96 where every field
+                                    starts in the phantom, else 32; 0xFFFFFFFF: no limit) */
+    uint32_t electron_chunk;     /* condensed-history steps per electron and sweep (picked by the run: 12 where every
+                                    field starts in the phantom, else 8; 0xFFFFFFFF: no limit) */
     uint32_t inject;             /* primaries injected per refill (6 Mi) */
     uint32_t threshold;          /* refill when fewer particles are in flight (6 Mi) */
     uint32_t sweeps_per_graph;   /* sweeps captured in one graph replay (4) */
@@ -169,8 +170,9 @@ typedef struct gegs_tuning {
                                     the electron side concurrently, 1 = one after the other (2) */
     uint32_t tail_particles;     /* once every source record is injected and at most this many particles are in
                                     flight, one launch finishes them, each with its descendants in one thread
-                                    (262144, the most; 0xFFFFFFFF: never, the sweeps run to the end); without
-                                    gegs_set_tuning a run of at most 8192 histories takes that launch at once */
+                                    (262144, the most; 0xFFFFFFFF: never, the sweeps run to the end); with
+                                    every field at its default a run of at most 8192 histories takes that
+                                    launch at once */
     uint64_t capacity;           /* particles per bank, rounded down to a multiple of 32: each bank is 32 equal
                                     append segments, and a full segment counts as overflow (0: twice the
                                     injection plus the threshold, each at most the run's histories, and at
@@ -356,8 +358,9 @@ int gegs_adjoint_device(gegs_ctx *ctx, const gegs_job *jobs, uint32_t n_jobs, ui
 int gegs_set_beamlet_weights_device(gegs_ctx *ctx, const float *weight, uint32_t n_beamlets);
 
 /* Tuning of gegs_run_event; NULL restores the defaults.  gegs_get_tuning
- * returns the values in force with defaults filled in (grid sizes that fill
- * the device are resolved at run time and reported as 0). */
+ * returns the values in force with defaults filled in; what each run picks
+ * (grid sizes that fill the device, and chunks and grid that the caller left
+ * to it) is reported as 0, and setting the returned values changes nothing. */
 int gegs_set_tuning(gegs_ctx *ctx, const gegs_tuning *tuning);
 int gegs_get_tuning(gegs_ctx *ctx, gegs_tuning *tuning);
 

@@ -194,7 +194,12 @@ def test_tuning_roundtrip_and_validation(gpu_ctx):
         gpu_ctx.set_tuning(dict(capacity=31))
     assert e.value.code == 2001
     gpu_ctx.set_tuning(None)
-    assert gpu_ctx.get_tuning()["photon_chunk"] == 32
+    base = gpu_ctx.get_tuning()
+    # the chunks and the interaction grid are each run's pick: no value to report
+    assert base["photon_chunk"] == base["electron_chunk"] == base["grid"] == 0
+    gpu_ctx.set_tuning(base)
+    assert gpu_ctx.get_tuning() == base
+    gpu_ctx.set_tuning(None)
 
 
 def test_batched_fields_and_plans_match_per_field_runs(gpu_ctx, ct_small):
