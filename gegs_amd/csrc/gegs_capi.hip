@@ -399,32 +399,44 @@ int gegs_set_history_tally(gegs_ctx *c, int enable) {
     return GEGS_OK;
 }
 
-// zeroed tallies for n_plans dose buffers and n_slots per-history slots
-static int prepare_tallies(gegs_ctx *c, uint32_t n_plans, uint64_t n_slots, uint32_t batch_rows = 1) {
+// zeroed tallies for n_plans dose buffers and n_slots per-history slots.
+// With `fewer` the run can do with fewer batch rows than asked for, and gets
+// there how many it has; the rows are reserved after everything else, so
+// that what a run cannot do without comes first.
+static int prepare_tallies(gegs_ctx *c, uint32_t n_plans, uint64_t n_slots, uint32_t batch_rows = 1,
+                           uint32_t *fewer = nullptr) {
     const size_t n = c->nvox * n_plans;
-    HIPCHECK(c, realloc_dev(c->d_chunk, c->chunk_n, n * batch_rows), "hipMalloc tally");
     size_t have = c->tally_n;
     HIPCHECK(c, realloc_dev(c->d_dose, have, n), "hipMalloc tally");
     have = c->tally_n;
     HIPCHECK(c, realloc_dev(c->d_dose2, have, n), "hipMalloc tally");
     if (c->tally_n < n) c->tally_n = n;
+    c->hist_len = c->hist_tally ? n_slots : 0;
+    if (c->hist_tally && c->hist_n < n_slots) {
+        hipFree(c->d_hist_edep);
+        hipFree(c->d_hist_steps);
+        c->d_hist_edep = nullptr;
+        c->d_hist_steps = nullptr;
+        HIPCHECK(c, hipMalloc(&c->d_hist_edep, n_slots * sizeof(double)), "hipMalloc history tally");
+        HIPCHECK(c, hipMalloc(&c->d_hist_steps, n_slots * sizeof(uint32_t)), "hipMalloc history tally");
+        c->hist_n = n_slots;
+    }
+    auto chunk = [&](uint32_t rows) { return realloc_dev(c->d_chunk, c->chunk_n, n * rows); };
+    if (fewer && c->chunk_n < n * batch_rows) {
+        size_t free = 0, total = 0;
+        HIPCHECK(c, hipMemGetInfo(&free, &total), "free memory");
+        HIPCHECK(c, reserve_rows(batch_rows, batch_rows, n, c->chunk_n * sizeof(double), free, chunk), "hipMalloc tally");
+    } else {
+        HIPCHECK(c, chunk(batch_rows), "hipMalloc tally");
+    }
+    if (fewer) *fewer = batch_rows;
     const int blocks = 2048;
     hipLaunchKernelGGL(fill_zero, dim3(blocks), dim3(256), 0, c->stream, c->d_chunk, n * batch_rows);
     hipLaunchKernelGGL(fill_zero, dim3(blocks), dim3(256), 0, c->stream, c->d_dose, n);
     hipLaunchKernelGGL(fill_zero, dim3(blocks), dim3(256), 0, c->stream, c->d_dose2, n);
     hipLaunchKernelGGL(fill_zero_u64, dim3(1), dim3(64), 0, c->stream, c->d_counters, (size_t)16);
     hipLaunchKernelGGL(fill_zero_u32, dim3(16), dim3(256), 0, c->stream, c->d_next, (size_t)4096);
-    c->hist_len = c->hist_tally ? n_slots : 0;
     if (c->hist_tally) {
-        if (c->hist_n < n_slots) {
-            hipFree(c->d_hist_edep);
-            hipFree(c->d_hist_steps);
-            c->d_hist_edep = nullptr;
-            c->d_hist_steps = nullptr;
-            HIPCHECK(c, hipMalloc(&c->d_hist_edep, n_slots * sizeof(double)), "hipMalloc history tally");
-            HIPCHECK(c, hipMalloc(&c->d_hist_steps, n_slots * sizeof(uint32_t)), "hipMalloc history tally");
-            c->hist_n = n_slots;
-        }
         hipLaunchKernelGGL(fill_zero, dim3(1024), dim3(256), 0, c->stream, c->d_hist_edep, (size_t)n_slots);
         hipLaunchKernelGGL(fill_zero_u32, dim3(1024), dim3(256), 0, c->stream, c->d_hist_steps, (size_t)n_slots);
     }
@@ -645,12 +657,6 @@ static int check_ready(gegs_ctx *c, const gegs_run_options *o) {
 // Batch rows held at once by a continuous run (bytes of per-batch dose rows).
 static constexpr size_t CONTINUOUS_TALLY_BYTES = (size_t)16 << 30;
 
-// dose rows of nvox doubles that fit `bytes`: at least one, at most one per batch
-static uint32_t batch_rows(size_t bytes, size_t nvox, uint32_t n_batches) {
-    const size_t fit = bytes / (nvox * sizeof(double));
-    return fit < 1 ? 1u : (fit < n_batches ? (uint32_t)fit : n_batches);
-}
-
 // the plain kernel instantiation for the record-table placement and the
 // options of the run (the general kernel for any of ENV_GENERAL)
 static void launch_plain(const PlainArgs &a, bool tab, uint32_t grid, uint32_t block, size_t lds, hipStream_t st) {
@@ -701,9 +707,6 @@ int gegs_run_plain(gegs_ctx *c, const gegs_run_options *o, double *dose, double 
     int rc = check_ready(c, o);
     if (rc) return rc;
     hipSetDevice(c->device);
-    const uint32_t rows = batch_rows(CONTINUOUS_TALLY_BYTES, c->nvox, o->n_batches);
-    rc = prepare_tallies(c, 1, c->nsrc, rows);
-    if (rc) return rc;
     rc = upload_jobs(c, {c->field}, {0u});
     if (rc) return rc;
     const uint32_t block = o->block_size ? o->block_size : PLAIN_BLOCK;
@@ -721,6 +724,10 @@ int gegs_run_plain(gegs_ctx *c, const gegs_run_options *o, double *dose, double 
     size_t have = c->stack_bytes / sizeof(float);
     HIPCHECK(c, realloc_dev(c->d_stack, have, nthreads * (size_t)depth * PART_WORDS), "hipMalloc stack");
     c->stack_bytes = have * sizeof(float);
+    // a row for every batch, or fewer rows and more launches where memory is short
+    uint32_t rows = batch_rows(CONTINUOUS_TALLY_BYTES, c->nvox, o->n_batches);
+    rc = prepare_tallies(c, 1, c->nsrc, rows, &rows);
+    if (rc) return rc;
     a.src = c->d_src;
     a.hist_offset = o->history_offset;
     a.stack = c->d_stack;

@@ -127,6 +127,29 @@ __host__ __device__ __forceinline__ uint32_t plain_lanes(uint64_t n, uint64_t wa
     return (uint32_t)(l < 1 ? 1 : (l > 64 ? 64 : l));
 }
 
+// dose rows of nvox doubles that fit `bytes`: at least one, at most one per batch
+inline uint32_t batch_rows(size_t bytes, size_t nvox, uint32_t n_batches) {
+    const size_t fit = bytes / (nvox * sizeof(double));
+    return fit < 1 ? 1u : (fit < n_batches ? (uint32_t)fit : n_batches);
+}
+
+// Memory for the dose rows of a run that can do with fewer than `want` of
+// them, one at least (its batches then take more launches): at most half of
+// what is free, where the `held` bytes of the context's rows count as free
+// and are kept in any case, and half as many again wherever that is refused.
+// `alloc(n)` makes room for n rows in place of those held.
+template <class Alloc>
+inline hipError_t reserve_rows(uint32_t &rows, uint32_t want, size_t nvox, size_t held, size_t free, Alloc alloc) {
+    const size_t half = (held >> 1) + (free >> 1);
+    rows = batch_rows(half > held ? half : held, nvox, want);
+    for (;;) {
+        const hipError_t e = alloc(rows);
+        if (e == hipSuccess || rows == 1) return e;
+        (void)hipGetLastError();
+        rows = (rows + 1) / 2;
+    }
+}
+
 template <bool TAB, bool GEN>
 __global__ void __launch_bounds__(128) GEGS_WAVES_PER_EU(2) plain_kernel(PlainArgs a) {
     extern __shared__ float lds_env[];
