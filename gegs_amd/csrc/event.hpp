@@ -82,6 +82,8 @@ struct EvState {
     QCount taken[N_SLOTS];           // work handed out from each bank (over its whole range)
 };
 
+constexpr uint32_t TAIL_BLOCK = 128;   // threads per block of the tail launch
+
 struct EventConfig {
     uint32_t block = 256;            // threads per block of the single-pass event kernels (<= 256)
     uint32_t flight_block = 256;     // threads per block of the photon and electron kernels (<= 512)
@@ -94,6 +96,7 @@ struct EventConfig {
     uint32_t refill_slots = 64;      // bank slots a wavefront reserves per refill atomic
     uint32_t sweep_streams = 2;      // 2: photon and electron sides of a sweep concurrently; 1: one after the other
     uint32_t tail = 1u << 18;        // in-flight particles that one tail launch finishes (0: no tail launch)
+    int tail_depth = 40;             // particles per thread's stack in that launch (the plain kernel's default)
     size_t capacity = 0;             // slots per bank (0: twice what can be in flight, at least 4 Mi)
     uint32_t inject = 6u << 20;      // primaries injected per refill
     uint32_t threshold = 6u << 20;   // refill when fewer particles are in flight
@@ -162,6 +165,20 @@ inline void pick_shape(EventConfig &cfg, bool head) {
     if (!cfg.photon_chunk) cfg.photon_chunk = head ? 32 : 96;
     if (!cfg.electron_chunk) cfg.electron_chunk = head ? 8 : 12;
     if (!cfg.grid) cfg.grid = 512;
+}
+
+// The tail launch of a run whose tables split photons (nbr_split photons per
+// bremsstrahlung and annihilation): its stacks are as much deeper as photons
+// are split, for as much fewer particles, so that they take the same memory
+// and overflow no sooner than without splitting.  Deepest stacks that
+// histories needed: CT 2e5 histories 5 unsplit, 32 at 8, 160 at 32; jaws and
+// MLC 1e5 histories 13, 81, 321.  Where less than a block's worth of
+// particles would be left, the sweeps run to the end.
+inline void split_tail(EventConfig &cfg, uint32_t nbr_split) {
+    if (nbr_split < 2) return;
+    cfg.tail /= nbr_split;
+    if (cfg.tail < TAIL_BLOCK) cfg.tail = 0;
+    else cfg.tail_depth *= (int)nbr_split;
 }
 
 // Source records of one batch, as slices of every job (field) of the run:
@@ -1177,7 +1194,6 @@ inline void launch_sweep(const EvArgs &a, const EventConfig &cfg, hipStream_t st
     else launch_sweep_f<false>(a, cfg, stream, t0, t1, f);
 }
 
-constexpr uint32_t TAIL_BLOCK = 128;
 // Histories of a run that the tail launch takes from the injection on, without
 // sweeps: up to 8192, 4 lanes of each resident wavefront.  A sweep of so few
 // particles takes as long as its slowest flight and there are at least 8
@@ -1186,7 +1202,6 @@ constexpr uint32_t TAIL_BLOCK = 128;
 // 2.35 -> 1.65 ms and through jaws and MLC 12.8 -> 9.1 ms; at 16 384 on the CT
 // 3.2 against 3.4 ms, at 70 001 3.3 against 4.8 ms.
 constexpr uint32_t TAIL_DIRECT = 8192;
-constexpr int TAIL_DEPTH = 40;       // particles per thread's stack (the plain kernel's default)
 
 // threads of the tail launch: one per particle up to `tail`, whole blocks
 inline uint32_t tail_threads(const EventConfig &cfg) {
@@ -1194,14 +1209,14 @@ inline uint32_t tail_threads(const EventConfig &cfg) {
 }
 
 // The tail launch and the bookkeeping after it; `stack` holds
-// tail_threads(cfg) x TAIL_DEPTH particles.
+// tail_threads(cfg) x cfg.tail_depth particles.
 template <bool TAB, bool ADJ, bool GEN>
 inline void launch_tail_t(const EvArgs &a, const EventConfig &cfg, float *stack, hipStream_t stream) {
     const uint32_t grid = tail_threads(cfg) / TAIL_BLOCK;
     const size_t lds = flight_lds(a.env);
     const uint32_t resident = resident_grid(tail_kernel<TAB, ADJ, GEN>, TAIL_BLOCK, lds);
     const uint32_t waves = (grid < resident ? grid : resident) * (TAIL_BLOCK / 64);
-    hipLaunchKernelGGL((tail_kernel<TAB, ADJ, GEN>), dim3(grid), dim3(TAIL_BLOCK), lds, stream, a, stack, TAIL_DEPTH,
+    hipLaunchKernelGGL((tail_kernel<TAB, ADJ, GEN>), dim3(grid), dim3(TAIL_BLOCK), lds, stream, a, stack, cfg.tail_depth,
                        waves);
 }
 
@@ -1345,7 +1360,7 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
     // most cfg.tail particles are in flight (not in a timed pass, whose
     // photon steps must all be photon-kernel steps).
     if (use_tail) {
-        const size_t need = (size_t)tail_threads(cfg) * TAIL_DEPTH * PART_WORDS;
+        const size_t need = (size_t)tail_threads(cfg) * (size_t)cfg.tail_depth * PART_WORDS;
         if (bk.tail_floats < need) {
             if (bk.tail_stack) (void)hipFree(bk.tail_stack);
             bk.tail_stack = nullptr;

@@ -33,6 +33,7 @@ struct gegs_ctx {
     bool odd_density = false;            // a density factor outside 2^-40 ... 2^40
     uint32_t max_med = 0;                // largest non-vacuum medium index of the phantom
     uint32_t nmed = 0;                   // media in the loaded tables
+    uint32_t nbr_split = 1;              // photons per bremsstrahlung and annihilation in the loaded tables
     float *d_xb = nullptr, *d_yb = nullptr, *d_zb = nullptr;
     uint32_t nx = 0, ny = 0, nz = 0;
     size_t nvox = 0;
@@ -215,6 +216,7 @@ int gegs_load_media(gegs_ctx *c, const gegs_media_tables *t) {
     HIPCHECK(c, hipMemcpyAsync(c->d_media, t, sizeof(gegs_media_tables), hipMemcpyHostToDevice, c->stream), "copy media");
     HIPCHECK(c, hipStreamSynchronize(c->stream), "sync media");
     c->nmed = (uint32_t)t->nmed;
+    c->nbr_split = (uint32_t)t->nbr_split;
     c->media_opts = (t->transport_algorithm == 0 ? ENV_PRESTA2 : 0u) | (t->exact_bca ? ENV_EXACT_BCA : 0u);
     c->have_media = true;
     return GEGS_OK;
@@ -901,6 +903,7 @@ static int run_event_jobs(gegs_ctx *c, const gegs_run_options *o, const std::vec
     bool head = false;
     for (const gegs_field &f : fields) head |= f.module_first != GEGS_M_PHANTOM;
     pick_shape(cfg, head);
+    split_tail(cfg, c->nbr_split);
     Env env = make_env(c, o->seed, (uint32_t)jobs.size());
     hipError_t e = c->banks.reserve(total_all, nb, cfg);
     if (e != hipSuccess) return fail(c, GEGS_ERR_DEVICE, "event banks", e);

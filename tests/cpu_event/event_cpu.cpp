@@ -199,7 +199,7 @@ int main(int argc, char **argv) {
     cfg.inject = m.inject ? m.inject : 256;
     cfg.threshold = m.threshold ? m.threshold : 512;
     cfg.tail = m.tail;
-    float *tail_stack = m.tail ? (float *)calloc((size_t)tail_threads(cfg) * TAIL_DEPTH * PART_WORDS, sizeof(float))
+    float *tail_stack = m.tail ? (float *)calloc((size_t)tail_threads(cfg) * (size_t)cfg.tail_depth * PART_WORDS, sizeof(float))
                                : nullptr;
     cpu_launch(batch_begin, dim3(1), dim3(1), st, 0u, m.nsrc, cfg.threshold, cfg.inject);
     bool tailed = false;

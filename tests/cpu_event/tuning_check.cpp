@@ -1,6 +1,7 @@
 // The caller's tuning and what a run makes of it (gegs_amd/csrc/event.hpp
-// config_of, tuning_of, pick_shape): a tuning read and set again leaves every
-// run's chunks, grid and short-run path as they were.
+// config_of, tuning_of, pick_shape, split_tail): a tuning read and set again
+// leaves every run's chunks, grid and short-run path as they were, and tables
+// that split photons get a tail with the stacks they need.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -57,6 +58,22 @@ int main() {
     a.refill_min = 9; a.refill_slots = 128; a.sweep_streams = 1; a.tail_particles = 99; a.capacity = 12345;
     const gegs_tuning b = tuning_of(config_of(a));
     check(memcmp(&a, &b, sizeof(a)) == 0, "every field given reads back");
+    // photons split n ways: stacks n times as deep for an n-th of the particles
+    for (uint32_t n : {1u, 2u, 3u, 8u, 32u, 2048u}) {
+        EventConfig c;
+        split_tail(c, n);
+        check(c.tail == d.tail / n && c.tail_depth == (int)(40u * n), "split tail");
+        check((uint64_t)tail_threads(c) * (uint64_t)c.tail_depth <= 3ull * tail_threads(d) * 40u / 2u, "split tail's memory");
+    }
+    for (uint32_t n : {2049u, 262145u, 0x7FFFFFFFu}) {
+        EventConfig c;
+        split_tail(c, n);
+        check(c.tail == 0, "split too far for a tail");
+    }
+    EventConfig few;
+    few.tail = 64;
+    split_tail(few, 1);
+    check(few.tail == 64 && few.tail_depth == 40, "a caller's short tail, unsplit");
     if (!fails) printf("ok\n");
     return fails != 0;
 }
