@@ -586,10 +586,6 @@ struct Refill {
     uint32_t next, end;      // wave-uniform reservation
     bool exhausted;
     uint32_t base;           // start of the range that `taken` hands out
-    __device__ __forceinline__ void init() {
-        next = end = base = 0;
-        exhausted = false;
-    }
     // The first 64 slots of each wavefront of the grid are its own, without
     // an atomic; `taken` hands out the rest.  When all 4 096 wavefronts took
     // their first slots from the one counter, a launch of the flight kernels

@@ -72,12 +72,12 @@ void k_push(EvArgs a) {
     }
 }
 
-// lanes take bank slots until the bank is exhausted, each lane keeping a
-// taken slot for (gid % 5) + 1 iterations
+// lanes take bank slots, their wavefront's own first, until the bank is
+// exhausted, each lane keeping a taken slot for (gid % 5) + 1 iterations
 void k_refill(uint32_t *taken, uint32_t n, uint32_t *hits, uint32_t min_idle) {
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     Refill rf;
-    rf.init();
+    rf.init_share(n);
     bool have = false;
     uint32_t left = 0;
     for (;;) {
@@ -150,14 +150,15 @@ int main(int argc, char **argv) {
         CHECK(st->overflow == 0);
         free(st);
     }
-    // refill reservations: every slot exactly once, for two thresholds
-    for (uint32_t min_idle : {1u, 16u}) {
-        const uint32_t n = 10007;
-        std::vector<uint32_t> hits(n, 0);
-        uint32_t taken = 0;
-        cpu_launch(k_refill, dim3(3), dim3(256), &taken, n, hits.data(), min_idle);
-        for (uint32_t i = 0; i < n; ++i) CHECK(hits[i] == 1u);
-    }
+    // refill reservations: every slot exactly once, for two thresholds, in
+    // banks from one particle to past the 768 slots of the wavefronts' shares
+    for (uint32_t min_idle : {1u, 16u})
+        for (uint32_t n : {1u, 63u, 65u, 767u, 768u, 769u, 10007u}) {
+            std::vector<uint32_t> hits(n, 0);
+            uint32_t taken = 0;
+            cpu_launch(k_refill, dim3(3), dim3(256), &taken, n, hits.data(), min_idle);
+            for (uint32_t i = 0; i < n; ++i) CHECK(hits[i] == 1u);
+        }
     printf("simt self-test: %d failures, %llu wavefront operations\n", failures, (unsigned long long)simt::S.ops);
     return failures ? 1 : 0;
 }
