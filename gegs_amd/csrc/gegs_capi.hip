@@ -1203,6 +1203,36 @@ int gegs_atomic_probe(gegs_ctx *c, const uint32_t *idx, uint64_t n, uint32_t nvo
     return GEGS_OK;
 }
 
+// Quotients and reciprocals of every mantissa: out[0] the quotients of the
+// logarithm (atanh_arg) that differ from the division, out[1] the largest
+// error of rcp_near, in units of 2^-32 of the value.
+static __global__ void reciprocal_probe(unsigned long long *out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // one thread per mantissa
+    const float m = __uint_as_float(0x3f3504f4u + i);
+    const float q = (m - 1.0f) / (m + 1.0f);
+    if (__float_as_uint(atanh_arg(m)) != __float_as_uint(q)) atomicAdd(out, 1ull);
+    const float x = __uint_as_float(0x3f800000u | i);
+    const double off = fabs(1.0 - (double)x * (double)rcp_near(x));
+    atomicMax(out + 1, (unsigned long long)(off * 4294967296.0));
+}
+
+int gegs_reciprocal_probe(gegs_ctx *c, uint64_t *quotients, double *reciprocal_ulps) {
+    if (!c || !quotients || !reciprocal_ulps) return fail(c, GEGS_ERR_ARG, "gegs_reciprocal_probe: bad argument");
+    hipSetDevice(c->device);
+    unsigned long long *d = nullptr, h[2] = {};
+    HIPCHECK(c, hipMalloc(&d, sizeof(h)), "hipMalloc probe");
+    hipLaunchKernelGGL(fill_zero_u64, dim3(1), dim3(64), 0, c->stream, d, (size_t)2);
+    hipLaunchKernelGGL(reciprocal_probe, dim3((1u << 23) / 256), dim3(256), 0, c->stream, d);
+    hipError_t e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = hipMemcpy(h, d, sizeof(h), hipMemcpyDeviceToHost);
+    hipFree(d);
+    if (e != hipSuccess) return fail(c, GEGS_ERR_DEVICE, "reciprocal probe", e);
+    *quotients = h[0];
+    // an ULP of a value in (1/2, 1] is 2^-24: at most 2^-23 of it
+    *reciprocal_ulps = (double)h[1] / 512.0;
+    return GEGS_OK;
+}
+
 int gegs_ct_subsize(int32_t size[3], int16_t *hu, const float voxel[3], float offset[3], const float box_min[3],
                     const float box_max[3]) {
     if (!size || !hu || !voxel || !offset || !box_min || !box_max) return GEGS_ERR_ARG;

@@ -23,8 +23,8 @@ __host__ __device__ __forceinline__ float pow2i(int k) {
 
 // (m - 1) / (m + 1) for m in [sqrt(1/2), sqrt(2)], correctly rounded.  On the
 // device the reciprocal, one product and one correction give the correctly
-// rounded quotient for every binary32 m of the interval (all 8 388 608
-// were compared with the division on gfx950; the scaling and special cases
+// rounded quotient for every binary32 m of the interval (gegs_reciprocal_probe
+// compares all 8 388 608 with the division; the scaling and special cases
 // of the general sequence are not needed there): 4 instructions for 11.
 __host__ __device__ __forceinline__ float atanh_arg(float m) {
 #if defined(__HIP_DEVICE_COMPILE__) && __HIP_DEVICE_COMPILE__

@@ -47,10 +47,13 @@ __device__ __forceinline__ P2 vtx(const gegs_float2 *poly, int i) { return p2(po
 // exit leaf left to the branches that use them), jaws and MLC 1e5 from 25.6 to
 // 22.9 ms.
 
-// 1/x to about 1 ULP, for the selections only (no result depends on it)
+// 1/x to about 1 ULP, for the selections only (no result depends on it).
+// The CPU check of the selections gives its own, as far off as the device's.
 __device__ __forceinline__ float rcp_near(float x) {
 #if defined(__HIP_DEVICE_COMPILE__) && __HIP_DEVICE_COMPILE__
     return __builtin_amdgcn_rcpf(x);
+#elif defined(GEGS_RCP_NEAR)
+    return GEGS_RCP_NEAR(x);
 #else
     return 1.0f / x;
 #endif

@@ -26,7 +26,7 @@ SYMBOLS = [
     "gegs_set_kernel_timing", "gegs_kernel_timing", "gegs_load_mlc", "gegs_set_leaf_positions",
     "gegs_load_jaws", "gegs_set_jaw_positions", "gegs_load_block_wedge", "gegs_set_fixes",
     "gegs_run_plain_noalloc", "gegs_run_batched_device", "gegs_adjoint_device",
-    "gegs_set_beamlet_weights_device",
+    "gegs_set_beamlet_weights_device", "gegs_reciprocal_probe",
 ]
 
 PARTICLE_DTYPE = np.dtype([("e", "<f4"), ("x", "<f4"), ("y", "<f4"), ("z", "<f4"), ("u", "<f4"),
@@ -121,6 +121,7 @@ def load():
     L.gegs_last_kernel_ms.argtypes = [vp, vp]
     L.gegs_sample_events.argtypes = [vp, vp, ctypes.c_uint32, ctypes.c_uint64, vp, ctypes.c_uint32, vp, vp]
     L.gegs_atomic_probe.argtypes = [vp, vp, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, vp]
+    L.gegs_reciprocal_probe.argtypes = [vp, vp, vp]
     L.gegs_ct_subsize.argtypes = [vp, vp, vp, vp, vp, vp]
     L.gegs_ct_resample_grid.argtypes = [vp, vp, vp, vp]
     L.gegs_ct_resample.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
@@ -256,6 +257,14 @@ class Context:
         ms = ctypes.c_float()
         self._check(self.L.gegs_atomic_probe(self.h, _p(idx), len(idx), int(nvox), int(reps), ctypes.byref(ms)))
         return reps * len(idx) / (ms.value * 1e-3)
+
+    def reciprocal_probe(self):
+        """(quotients of the device's logarithm that differ from the division,
+        largest error of the reciprocal that chooses polygon edges in units of
+        2^-23 of the value), over all mantissas (gegs_reciprocal_probe)."""
+        n, ulps = ctypes.c_uint64(), ctypes.c_double()
+        self._check(self.L.gegs_reciprocal_probe(self.h, ctypes.byref(n), ctypes.byref(ulps)))
+        return int(n.value), float(ulps.value)
 
     def sample_events(self, particles, seed, max_out=16):
         """Run one event handler per particle (PARTICLE_DTYPE records);

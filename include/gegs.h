@@ -399,6 +399,15 @@ int gegs_kernel_timing(gegs_ctx *ctx, double *photon_ms, uint64_t *photon_launch
  * (escore's FP64 atomicAdd, scoring.cu:14-24, utility.cu:52-61). */
 int gegs_atomic_probe(gegs_ctx *ctx, const uint32_t *idx, uint64_t n, uint32_t nvox, uint32_t reps, float *ms);
 
+/* The device forms of the arithmetic that starts from the hardware's
+ * reciprocal, over all 2^23 mantissas: *quotients counts the logarithm's
+ * quotients (m - 1) / (m + 1), m in [sqrt(1/2), sqrt(2)], that are not the
+ * correctly rounded ones (results equal the oracle's where it is 0), and
+ * *reciprocal_ulps is the largest error, in units of 2^-23 of the value, of
+ * the reciprocal that only chooses polygon edges.  Diagnostics; no
+ * counterpart in the reference. */
+int gegs_reciprocal_probe(gegs_ctx *ctx, uint64_t *quotients, double *reciprocal_ulps);
+
 /* CT front end (host only, no device or context needed).  Volumes of CT
  * numbers are x-fastest int16: hu[i + nx * (j + ny * k)]; lengths in cm.
  *

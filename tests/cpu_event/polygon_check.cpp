@@ -1,7 +1,8 @@
 // The polygon tests of the head geometry (gegs_amd/csrc/mlc.hpp) against their
 // plain forms: every edge divided and every distance rooted, as the
 // reference writes them (geom.cu:310-327, :442-484, :1152-1191).  Results
-// must be equal bit for bit.  argv[1]: number of random polygons.
+// must be equal bit for bit.  argv[1]: number of random polygons; argv[2]: how
+// many ULP the reciprocals that the selections use are off at most (0: none).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -11,6 +12,17 @@
 #include <random>
 #include <vector>
 
+// a reciprocal as far off as the device's, up or down, another way each call
+static unsigned rcp_ulps = 0;
+static float rcp_off(float x) {
+    const float y = 1.0f / x;
+    if (!rcp_ulps || !(fabsf(y) >= 1.17549435e-38f && fabsf(y) <= 1e38f)) return y;
+    static uint32_t state = 12345u;
+    state = state * 1664525u + 1013904223u;
+    const int d = (int)((state >> 16) % (2u * rcp_ulps + 1u)) - (int)rcp_ulps;
+    return __uint_as_float((uint32_t)((int64_t)__float_as_uint(y) + d));
+}
+#define GEGS_RCP_NEAR rcp_off
 #include "../../gegs_amd/csrc/event.hpp"
 
 namespace gegs {
@@ -73,6 +85,7 @@ static bool same(float a, float b) { return memcmp(&a, &b, 4) == 0 || (a == 0.0f
 
 int main(int argc, char **argv) {
     const int polys = argc > 1 ? atoi(argv[1]) : 1000;
+    rcp_ulps = argc > 2 ? (unsigned)atoi(argv[2]) : 0u;
     std::mt19937 rng(5);
     auto uni = [&](float lo, float hi) { return lo + (hi - lo) * (float)(rng() >> 8) * (1.0f / 16777216.0f); };
     size_t checks = 0, hits = 0;

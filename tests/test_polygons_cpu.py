@@ -3,7 +3,8 @@ edge, distance to the nearest edge), which pick the deciding edge with cheap
 arithmetic, against their plain forms, compiled for the CPU: bit for bit over
 slabs, leaves, leaf ends and random polygons (lengths 1e-3 to 1e4 cm, edges
 of no length), with points on and beside vertices and edges and directions
-along the axes, at vertices and near zero."""
+along the axes, at vertices and near zero.  The device's own reciprocals and
+quotients are checked by test_gpu_reciprocals.py."""
 import os
 import subprocess
 
@@ -18,9 +19,11 @@ def test_polygon_tests_equal_their_plain_forms(tmp_path):
     exe = str(tmp_path / "polygon_check")
     subprocess.check_call([CLANG, "-std=c++17", "-O2", "-ffp-contract=off", "-I", os.path.join(HERE, "cpu_event", "include"),
                            "-DLDS_FLOATS=1", "-o", exe, os.path.join(HERE, "cpu_event", "polygon_check.cpp")])
-    r = subprocess.run([exe, "6000"], capture_output=True, text=True, timeout=600)
-    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
-    assert r.stdout.startswith("checks 2400000")
+    # the selections' reciprocals exact, as far off as the device's (1 ULP) and twice as far
+    for ulps in ("0", "1", "2"):
+        r = subprocess.run([exe, "6000", ulps], capture_output=True, text=True, timeout=600)
+        assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+        assert r.stdout.startswith("checks 2400000")
 
 
 def test_walk_quotients_and_logarithm_equal_their_plain_forms(tmp_path):
