@@ -1196,7 +1196,9 @@ inline void launch_sweep(const EvArgs &a, const EventConfig &cfg, hipStream_t st
 // (two graph replays).  Kernel time with and without the sweeps: 1 000
 // histories on the CT 2.6 -> 1.5 ms, 4 096 2.8 -> 2.2 ms, 10 001 on water
 // 2.35 -> 1.65 ms and through jaws and MLC 12.8 -> 9.1 ms; at 16 384 on the CT
-// 3.2 against 3.4 ms, at 70 001 3.3 against 4.8 ms.
+// 3.2 against 3.4 ms, at 70 001 3.3 against 4.8 ms.  A line at 16 384 for all
+// runs was mixed: 16 001 histories on water 2.1 -> 1.7 ms and through jaws and
+// MLC 12.5 -> 11.6, on the CT 3.8 -> 3.9, with PRESTA-II 3.7 -> 3.9.
 constexpr uint32_t TAIL_DIRECT = 8192;
 
 // threads of the tail launch: one per particle up to `tail`, whole blocks

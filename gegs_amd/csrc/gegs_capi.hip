@@ -752,7 +752,10 @@ int gegs_run_plain(gegs_ctx *c, const gegs_run_options *o, double *dose, double 
 
 // Part of the no-alloc scratch that may hold dose rows of several batches; the
 // rest is for particle stacks (a 128x128x100 CT's five rows leave 616 blocks
-// of 40-deep stacks, one row 778).
+// of 40-deep stacks, one row 778).  The launches saved are worth more than the
+// blocks lost at every length there, ten batches, ms: 1 001 histories 2.2
+// against 8.7 with one row, 1e4 4.2 against 12.5, 1e5 9.7 against 25.4, 1e6
+// 40.8 against 53.1 (five batches, one launch against five: 37.2 against 42.7).
 static constexpr size_t NOALLOC_ROW_BYTES = GEGS_NOALLOC_SCRATCH_BYTES / 4;
 
 // Layout of the no-alloc scratch for a run on nvox voxels: counters, batch
