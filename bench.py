@@ -496,7 +496,8 @@ def main():
             if timing and timing[1]:
                 photon_ms, launches = timing
                 pbytes = PHOTON_STEP_BYTES * cnt2["photon_steps"]
-                per_step = measured_traffic_per_photon_step()
+                # counted at the chunks the library picks: suspended flights are part of the traffic
+                per_step = measured_traffic_per_photon_step() if not ctx.get_tuning()["photon_chunk"] else None
                 res["roofline"] = dict(kernel="photon_kernel", launches=launches,
                                        traffic=(per_step * cnt2["photon_steps"] / launches) if per_step else None,
                                        avg_launch_us=photon_ms / launches * 1e3,
@@ -555,7 +556,8 @@ def main():
         roof = {"bound": "hbm", "achieved": rf["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": rf["achieved"] / HBM_PEAK_GBS, "traffic": rf["traffic"], "kernel": rf["kernel"],
                 "traffic_source": "profiles/photon_kernel_ct128_event.md: rocprofv3 FETCH_SIZE x2 + WRITE_SIZE x1 "
-                                  "(1 GiB copy calibration) per photon step, times this run's photon steps per launch",
+                                  "(1 GiB copy calibration) per photon step at the library's own chunks, times this run's "
+                                  "photon steps per launch (null under another photon_chunk)",
                 "avg_launch_us": rf["avg_launch_us"], "launches": rf["launches"],
                 "algorithmic_bytes_per_launch": rf["algorithmic_bytes_per_launch"],
                 "algorithmic_bytes_per_photon_step": PHOTON_STEP_BYTES,
