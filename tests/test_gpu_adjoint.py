@@ -88,10 +88,16 @@ def test_adjoint_matches_influence_matrix(gpu_ctx, ct):
     m, p = _objective(ct, d_ref)
     dLdD = 2.0 * m * (d_ref - p)
     g_ref = A[:, :plan.n_beamlets].T @ dLdD
-    d = plan.forward(w)
-    assert np.allclose(d, d_ref, rtol=1e-5, atol=1e-9 * d_ref.max())
-    g = plan.adjoint(dLdD)
-    assert np.allclose(g, g_ref, rtol=1e-9, atol=1e-12 * np.abs(g_ref).max())
+    try:
+        # the whole run in the tail launch (the default at this size), and the sweeps to the end
+        for tuning in (None, dict(tail_particles=0xFFFFFFFF)):
+            gpu_ctx.set_tuning(tuning)
+            d = plan.forward(w)
+            assert np.allclose(d, d_ref, rtol=1e-5, atol=1e-9 * d_ref.max())
+            g = plan.adjoint(dLdD)
+            assert np.allclose(g, g_ref, rtol=1e-9, atol=1e-12 * np.abs(g_ref).max())
+    finally:
+        gpu_ctx.set_tuning(None)
     gpu_ctx.set_beamlets(None)
 
 

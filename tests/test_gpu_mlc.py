@@ -46,11 +46,18 @@ def test_mlc_event_matches_plain(gpu_ctx, ct_mlc):
     src = ct_mlc.source(6000, 4)
     _load(gpu_ctx, ct_mlc, src)
     p = gpu_ctx.run(seed=5, n_batches=2, method="plain", per_history=True)
+    gpu_ctx.set_tuning(None)
     e = gpu_ctx.run(seed=5, n_batches=2, method="event", per_history=True)
-    assert e["counters"]["overflow"] == 0
-    assert np.array_equal(e["steps"], p["steps"])
-    assert np.array_equal(e["edep"], p["edep"])
-    assert np.allclose(e["dose"], p["dose"], rtol=1e-11, atol=1e-12)
+    gpu_ctx.set_tuning(tail_particles=0xFFFFFFFF)     # the sweeps to the end, which so short a run otherwise skips
+    try:
+        w = gpu_ctx.run(seed=5, n_batches=2, method="event", per_history=True)
+    finally:
+        gpu_ctx.set_tuning(None)
+    for r in (e, w):
+        assert r["counters"]["overflow"] == 0
+        assert np.array_equal(r["steps"], p["steps"])
+        assert np.array_equal(r["edep"], p["edep"])
+        assert np.allclose(r["dose"], p["dose"], rtol=1e-11, atol=1e-12)
 
 
 def test_mlc_leaf_sets_per_job(gpu_ctx, ct_mlc):
@@ -67,9 +74,13 @@ def test_mlc_leaf_sets_per_job(gpu_ctx, ct_mlc):
     try:
         jobs = [dict(field=f0, plan=0, first=0, count=3000, leaf_set=0),
                 dict(field=f1, plan=1, first=3000, count=2000, leaf_set=1)]
+        gpu_ctx.set_tuning(None)
         bt = gpu_ctx.run_batched(jobs, 2, seed=23, n_batches=2, per_history=True)
-        assert bt["counters"]["overflow"] == 0
+        gpu_ctx.set_tuning(tail_particles=0xFFFFFFFF)     # the sweeps to the end, which so short a run otherwise skips
+        sw = gpu_ctx.run_batched(jobs, 2, seed=23, n_batches=2, per_history=True)
+        assert bt["counters"]["overflow"] == 0 and sw["counters"]["overflow"] == 0
     finally:
+        gpu_ctx.set_tuning(None)
         gpu_ctx.set_leaf_positions(ct_mlc.leaf_positions)
     for jb, pos in ((jobs[0], ct_mlc.leaf_positions), (jobs[1], pos2)):
         wl = copy.copy(ct_mlc)
@@ -77,8 +88,9 @@ def test_mlc_leaf_sets_per_job(gpu_ctx, ct_mlc):
         wl.leaf_positions = pos
         sl = slice(jb["first"], jb["first"] + 600)
         o = oracle.run(wl, src[sl], seed=23, hist_offset=jb["first"], per_history=True)
-        assert np.array_equal(bt["steps"][sl], o["steps"])
-        assert np.array_equal(bt["edep"][sl], o["edep"])
+        for r in (bt, sw):
+            assert np.array_equal(r["steps"][sl], o["steps"])
+            assert np.array_equal(r["edep"][sl], o["edep"])
 
 
 def test_jaws_then_mlc_bit_exact(gpu_ctx):
@@ -90,12 +102,17 @@ def test_jaws_then_mlc_bit_exact(gpu_ctx):
     _load(gpu_ctx, wl, src)
     try:
         g = gpu_ctx.run(seed=31, n_batches=2, method="plain", per_history=True)
+        gpu_ctx.set_tuning(None)
         e = gpu_ctx.run(seed=31, n_batches=2, method="event", per_history=True)
+        gpu_ctx.set_tuning(tail_particles=0xFFFFFFFF)     # the sweeps to the end, which so short a run otherwise skips
+        w = gpu_ctx.run(seed=31, n_batches=2, method="event", per_history=True)
     finally:
+        gpu_ctx.set_tuning(None)
         gpu_ctx.set_field(workloads.ct_mlc().field)
     o = oracle.run(wl, src, seed=31, per_history=True)
     assert np.array_equal(g["steps"], o["steps"])
     assert np.array_equal(g["edep"], o["edep"])
-    assert np.array_equal(e["steps"], g["steps"])
-    assert np.allclose(e["edep"], g["edep"], rtol=1e-12, atol=1e-12)
-    assert e["counters"]["overflow"] == 0
+    for r in (e, w):
+        assert np.array_equal(r["steps"], g["steps"])
+        assert np.allclose(r["edep"], g["edep"], rtol=1e-12, atol=1e-12)
+        assert r["counters"]["overflow"] == 0

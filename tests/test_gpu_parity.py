@@ -217,8 +217,17 @@ def test_batched_fields_and_plans_match_per_field_runs(gpu_ctx, ct_small):
     jobs = [dict(field=fields[0], plan=0, first=0, count=3000),
             dict(field=fields[1], plan=1, first=3000, count=2000),
             dict(field=fields[2], plan=0, first=5000, count=1000)]
+    gpu_ctx.set_tuning(None)
     bt = gpu_ctx.run_batched(jobs, 2, seed=11, n_batches=3, per_history=True)
-    assert bt["counters"]["overflow"] == 0
+    gpu_ctx.set_tuning(tail_particles=0xFFFFFFFF)     # the sweeps to the end, which so short a run otherwise skips
+    try:
+        sw = gpu_ctx.run_batched(jobs, 2, seed=11, n_batches=3, per_history=True)
+    finally:
+        gpu_ctx.set_tuning(None)
+    assert bt["counters"]["overflow"] == 0 and sw["counters"]["overflow"] == 0
+    assert np.array_equal(sw["steps"], bt["steps"])
+    assert np.allclose(sw["edep"], bt["edep"], rtol=1e-12, atol=1e-12)
+    assert np.allclose(sw["dose"], bt["dose"], rtol=1e-11, atol=1e-12)
     ref_dose = np.zeros((2, gpu_ctx.nvox))
     slot = 0
     try:
