@@ -72,8 +72,10 @@ def autotune(ctx, first, count, seed=1, repeat=2, tol=0.02, rounds=1, log=None):
                 if r > best * (1.0 + tol):
                     best, cur = r, t
     if cur != START:
-        base = _rate(ctx, START, first, count, seed, repeat)
-        again = _rate(ctx, cur, first, count, seed, repeat)
+        # in turn, the defaults first and last, so that a drift of the
+        # machine's speed does not pass for a gain
+        at = [_rate(ctx, t, first, count, seed, repeat + 1) for t in (START, cur, cur, START)]
+        base, again = max(at[0], at[3]), max(at[1], at[2])
         trials += [(dict(START), base), (dict(cur), again)]
         best = again
         if again <= base * (1.0 + tol):

@@ -58,3 +58,10 @@ def test_one_lucky_trial_is_not_kept(monkeypatch):
         return 0.5 if _given(t) == dict(electron_chunk=32) and c.runs.count(c.tuning) <= 2 else 1.0
     ctx, tuning, best, _ = _tune(monkeypatch, cost)
     assert _given(tuning) == {} and best == 1000.0
+
+
+def test_a_drift_of_the_machine_is_not_a_gain(monkeypatch):
+    """Every run a little faster than the one before, whatever the tuning: the
+    later trials win, and lose against the defaults timed before and after them."""
+    ctx, tuning, best, _ = _tune(monkeypatch, lambda c, t: 0.985 ** len(c.runs))
+    assert _given(tuning) == {}
