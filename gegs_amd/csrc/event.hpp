@@ -168,17 +168,23 @@ inline void pick_shape(EventConfig &cfg, bool head) {
 }
 
 // The tail launch of a run whose tables split photons (nbr_split photons per
-// bremsstrahlung and annihilation): its stacks are as much deeper as photons
-// are split, for as much fewer particles, so that they take the same memory
-// and overflow no sooner than without splitting.  Deepest stacks that
-// histories needed: CT 2e5 histories 5 unsplit, 32 at 8, 160 at 32; jaws and
-// MLC 1e5 histories 13, 81, 321.  Where less than a block's worth of
-// particles would be left, the sweeps run to the end.
+// bremsstrahlung and annihilation): stacks as much deeper as photons are
+// split, so that they overflow no sooner than without splitting.  Deepest
+// stacks that histories needed: CT 2e5 histories 5 unsplit, 32 at 8, 160 at
+// 32; jaws and MLC 1e5 histories 13, 81, 321.  Past 8 photons the launch takes
+// as much fewer particles, which keeps the stacks at 8 times their memory
+// (5.4 GB; fewer particles from 2 photons on took 671 MB throughout and 3e5
+// histories on water from 3.6 to 4.2 ms at 4 photons, from 3.9 to 4.8 at 8).
+// Where less than a block's worth of particles would be left, the sweeps run
+// to the end.
+constexpr uint32_t SPLIT_DEEPER = 8;
 inline void split_tail(EventConfig &cfg, uint32_t nbr_split) {
     if (nbr_split < 2) return;
-    cfg.tail /= nbr_split;
-    if (cfg.tail < TAIL_BLOCK) cfg.tail = 0;
-    else cfg.tail_depth *= (int)nbr_split;
+    if (nbr_split > SPLIT_DEEPER) {
+        cfg.tail = (uint32_t)((uint64_t)cfg.tail * SPLIT_DEEPER / nbr_split);
+        if (cfg.tail < TAIL_BLOCK) cfg.tail = 0;
+    }
+    if (cfg.tail) cfg.tail_depth *= (int)nbr_split;
 }
 
 // Source records of one batch, as slices of every job (field) of the run:
@@ -1332,7 +1338,26 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
     // group is captured once per argument set and replayed.
     const bool timed = bk.timing && cfg.sweeps_per_graph <= (uint32_t)EventBanks::MAX_TIMED;
     const SweepFork fork = cfg.sweep_streams == 2 ? bk.fork : SweepFork();
-    const bool use_tail = cfg.tail && !timed;
+    // The tail launch finishes the run once every record is injected and at
+    // most cfg.tail particles are in flight (not in a timed pass, whose
+    // photon steps must all be photon-kernel steps).  Without memory for its
+    // stacks the sweeps run to the end.
+    bool use_tail = cfg.tail && !timed;
+    if (use_tail) {
+        const size_t need = (size_t)tail_threads(cfg) * (size_t)cfg.tail_depth * PART_WORDS;
+        if (bk.tail_floats < need) {
+            if (bk.tail_stack) (void)hipFree(bk.tail_stack);
+            bk.tail_stack = nullptr;
+            bk.tail_floats = 0;
+            if (hipMalloc(&bk.tail_stack, need * sizeof(float)) == hipSuccess) {
+                bk.tail_floats = need;
+            } else {
+                (void)hipGetLastError();
+                bk.tail_stack = nullptr;
+                use_tail = false;
+            }
+        }
+    }
     // a run this short goes to the tail launch at once: no sweeps, no graph
     const uint32_t total = bk.h_plan->total;
     const bool direct = use_tail && cfg.direct && total <= TAIL_DIRECT && total <= cfg.inject && total <= cfg.tail;
@@ -1353,20 +1378,6 @@ inline hipError_t run_event_batch(EventBanks &bk, const Env &env, const gegs_sou
         if (e != hipSuccess) return e;
         bk.graph_args = a;
         bk.graph_cfg = cfg;
-    }
-    // The tail launch finishes the run once every record is injected and at
-    // most cfg.tail particles are in flight (not in a timed pass, whose
-    // photon steps must all be photon-kernel steps).
-    if (use_tail) {
-        const size_t need = (size_t)tail_threads(cfg) * (size_t)cfg.tail_depth * PART_WORDS;
-        if (bk.tail_floats < need) {
-            if (bk.tail_stack) (void)hipFree(bk.tail_stack);
-            bk.tail_stack = nullptr;
-            bk.tail_floats = 0;
-            e = hipMalloc(&bk.tail_stack, need * sizeof(float));
-            if (e != hipSuccess) return e;
-            bk.tail_floats = need;
-        }
     }
     e = hipMemcpyAsync(bk.d_plan, bk.h_plan, sizeof(BatchPlan), hipMemcpyHostToDevice, stream);
     if (e != hipSuccess) return e;

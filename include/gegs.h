@@ -172,7 +172,7 @@ typedef struct gegs_tuning {
                                     flight, one launch finishes them, each with its descendants in one thread
                                     (262144, the most; 0xFFFFFFFF: never, the sweeps run to the end); with
                                     every field at its default a run of at most 8192 histories takes that
-                                    launch at once; tables that split photons n ways (nbr_split): an n-th of
+                                    launch at once; for tables that split photons n > 8 ways (nbr_split) 8/n of
                                     the particles, never where that is below 128 */
     uint64_t capacity;           /* particles per bank, rounded down to a multiple of 32: each bank is 32 equal
                                     append segments, and a full segment counts as overflow (0: twice the

@@ -58,14 +58,14 @@ int main() {
     a.refill_min = 9; a.refill_slots = 128; a.sweep_streams = 1; a.tail_particles = 99; a.capacity = 12345;
     const gegs_tuning b = tuning_of(config_of(a));
     check(memcmp(&a, &b, sizeof(a)) == 0, "every field given reads back");
-    // photons split n ways: stacks n times as deep for an n-th of the particles
-    for (uint32_t n : {1u, 2u, 3u, 8u, 32u, 2048u}) {
+    // photons split n ways: stacks n times as deep, past 8 for 8/n of the particles
+    for (uint32_t n : {1u, 2u, 3u, 8u, 9u, 32u, 16384u}) {
         EventConfig c;
         split_tail(c, n);
-        check(c.tail == d.tail / n && c.tail_depth == (int)(40u * n), "split tail");
-        check((uint64_t)tail_threads(c) * (uint64_t)c.tail_depth <= 3ull * tail_threads(d) * 40u / 2u, "split tail's memory");
+        check(c.tail == (n <= 8u ? d.tail : d.tail * 8u / n) && c.tail_depth == (int)(40u * n), "split tail");
+        check((uint64_t)tail_threads(c) * (uint64_t)c.tail_depth <= 8ull * tail_threads(d) * 40u * 3u / 2u, "split tail's memory");
     }
-    for (uint32_t n : {2049u, 262145u, 0x7FFFFFFFu}) {
+    for (uint32_t n : {16385u, 262145u, 0x7FFFFFFFu}) {
         EventConfig c;
         split_tail(c, n);
         check(c.tail == 0, "split too far for a tail");
