@@ -478,8 +478,9 @@ def main():
         tuning = json.loads(args.tuning)
         ctx.set_tuning(tuning)
     elif "event" in methods and not args.no_autotune:
-        # tuned on the warmup records, before the timed region
-        tuning, _, _ = autotune.autotune(ctx, 0, min(max(args.warmup, 1) * b, 2_000_000), seed=args.seed, repeat=3)
+        # tuned before the timed region, on runs as long as the timed one (up to 1e7 records):
+        # photon chunk 64 is 3% faster than the default for 1e6 histories and 2% slower for 1e7
+        tuning, _, _ = autotune.autotune(ctx, 0, min(args.steps * b, 10_000_000), seed=args.seed, repeat=3)
     results = {}
     for method in methods:
         elapsed, dose, dose2, cnt, _ = run_method(ctx, method, args.steps, args.warmup, b, args.seed)

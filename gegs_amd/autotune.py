@@ -49,7 +49,8 @@ def _rate(ctx, tuning, first, count, seed, repeat):
 
 def autotune(ctx, first, count, seed=1, repeat=2, tol=0.02, rounds=1, log=None):
     """Tune the event method on source records [first, first+count) of the
-    loaded context.  Returns (tuning dict, histories/s of its last trial,
+    loaded context, which should be as many as the runs it is for: what is best
+    moves with the run's length.  Returns (tuning dict, histories/s of its last trial,
     list of (tuning, histories/s) trials).  The context keeps that tuning."""
     cur = dict(START)
     trials = []
