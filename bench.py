@@ -217,7 +217,7 @@ def mlc_plan_bench(n_total, n_batches, seed, autotune_first=True, fixed_tuning=N
     elif autotune_first:
         ctx.set_leaf_positions(plan.leaf_positions[0])
         ctx.set_field(plan.fields[0])
-        tuning, _, _ = autotune.autotune(ctx, 0, min(int(plan.counts(n_total)[0]), 1_000_000), seed=seed, repeat=3)
+        tuning, _, _ = autotune.autotune(ctx, 0, min(int(plan.counts(n_total)[0]), 10_000_000), seed=seed, repeat=3)
     jobs = plan.jobs(n_total)
     out = {}
     # warm-up: graph capture and first launches on a small slice
